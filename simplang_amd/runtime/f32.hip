@@ -581,6 +581,19 @@ int dispatch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, i
   if (!ok) return 1;
   const int64_t cus = num_cus();
   auto tiles = [&](int bm, int bn) { return cdiv(M, bm) * cdiv(N, bn) * batch; };
+  // one round of 64x64 ring tiles with a short K stays ahead of the split
+  // products' larger tiles (200x256x4096 8.3 us against 9.7, 512x768x2048 18.4
+  // against 19.6; 300x256x4096 12.9 against 9.9, 512x2048x2048 43 against 32)
+  const int64_t t64 = tiles(64, 64);
+  const bool one_round = K % 32 == 0 && K <= 1024 && t64 >= cus && 8 * t64 <= 9 * cus;
+  // products of about a MB of weights likewise (two launches either way):
+  // 24x768x768 9.2 us against 9.8, 128x768x768 with B_T 10.5 against 11.4
+  const int64_t kn = (int64_t)K * N;
+  const bool small = M <= 32 ? kn < (1 << 20) : BT && M <= 128 && kn <= (5 << 18);
+  if (batch == 1 && M > 16 && !one_round && !small) {
+    const int rc = launch_x3_f32(BT, A, lda, B, ldb, C, ldc, M, N, K, beta, false, st);
+    if (rc != 1) return rc;
+  }
   if (M <= 16)
     return launch_mfma_f32<16, 256, 1, 4, BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, batch, beta, st);
   if (M <= 32)
@@ -630,6 +643,12 @@ int launch_gemm_t(const T *A, int64_t lda, int64_t sa, const T *B, int64_t ldb, 
     if (batch <= 65535) {
       const int rc = dispatch_mfma_f32<BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, (int)batch,
                                            beta, st);
+      if (rc != 1) return rc;
+    }
+  }
+  if constexpr (std::is_same<T, float>::value) {
+    if (batch == 1) {
+      const int rc = launch_x3_f32(BT, A, lda, B, ldb, C, ldc, M, N, K, beta, true, st);
       if (rc != 1) return rc;
     }
   }

@@ -1,0 +1,598 @@
+// gemm_x3.hip -- fp32 and W4 matrix products on the bf16 matrix cores.
+//
+// Every fp32 operand is split into three bf16 parts, x = h + m + l exactly (8 +
+// 8 + 8 significant bits: h = bf16(x), m = bf16(x - h), l = x - h - m), whose
+// products are exact in fp32.  A product of two fp32 values keeps the six parts
+// hh, hm, mh, hl, lh and mm; the three dropped ones are below 2^-25 of it, less
+// than one fp32 rounding.  A W4 weight is one exact bf16, so there the three
+// products are all of them.  v_mfma_f32_16x16x32_bf16 runs at 16 times the rate
+// of v_mfma_f32_16x16x4_f32 and rounds its accumulator once per 32 products
+// instead of once per 4, so six of them are faster than the fp32 MFMA and no
+// less exact.
+#include <algorithm>
+#include <type_traits>
+
+#include "rt_device.h"
+#include "rt_internal.h"
+
+namespace simp {
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+// 16-byte loads and stores of floats that are only 4-byte aligned (odd leading
+// dimensions): the type says so, and the compiler picks the instruction.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+
+enum { kBKN = 0, kBNK = 1, kBW4 = 2 };  // B[K,N], B_T[N,K], W4 rows [N, K/2]
+
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  const f2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
+}
+
+struct Planes {
+  b8 h, m, l;
+};
+
+// The matrix cores flush bf16 subnormals, which the low parts of an x below
+// 2^-102 would be.  So x is scaled by 2^24 first (exact; the sums are scaled
+// back at the end): every fp32 value down to the subnormals keeps its 24 bits,
+// and one above 2^103 overflows into the non-finite sums that are formed again
+// in fp32.
+constexpr float kUp = 16777216.f;
+
+// The three bf16 parts of eight floats, scaled by kUp.
+__device__ __forceinline__ Planes split8(const float (&x)[8]) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float x0 = kUp * x[2 * i], x1 = kUp * x[2 * i + 1];
+    h[i] = pk_bf16(x0, x1);
+    const float r0 = x0 - __uint_as_float(h[i] << 16), r1 = x1 - __uint_as_float(h[i] & 0xFFFF0000u);
+    m[i] = pk_bf16(r0, r1);
+    l[i] = pk_bf16(r0 - __uint_as_float(m[i] << 16), r1 - __uint_as_float(m[i] & 0xFFFF0000u));
+  }
+  Planes p;
+  p.h = __builtin_bit_cast(b8, make_uint4(h[0], h[1], h[2], h[3]));
+  p.m = __builtin_bit_cast(b8, make_uint4(m[0], m[1], m[2], m[3]));
+  p.l = __builtin_bit_cast(b8, make_uint4(l[0], l[1], l[2], l[3]));
+  return p;
+}
+
+// Eight signed nibbles (low nibble first) as bf16 sixteenths: v_cvt_off_f32_i4
+// gives q / 16, exact in the upper half of its fp32 form.  The caller's scale
+// carries the 16.
+__device__ __forceinline__ b8 nib8_bf16(uint32_t w) {
+  const uint32_t v = w >> 4;
+  uint32_t p[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float lo = __builtin_amdgcn_cvt_off_f32_i4(w >> (8 * i));
+    const float hi = __builtin_amdgcn_cvt_off_f32_i4(v >> (8 * i));
+    p[i] = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+  }
+  return __builtin_bit_cast(b8, make_uint4(p[0], p[1], p[2], p[3]));
+}
+
+__device__ __forceinline__ v4f mfma_bf16(b8 a, b8 b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+struct X3Args {
+  const float *A;
+  int64_t lda;
+  const void *B;
+  int64_t ldb;       // floats; bytes for W4
+  const float *S;    // W4 scales [N, lds], one per `cpg` groups of 32
+  int64_t lds;
+  int cpg, cpg_shift;
+  float *C;
+  int64_t ldc;
+  float *P;          // partial products [split][M][N]; null: straight to C
+  int M, N, K;
+  int span;          // K steps of 32 per split
+  int tiles_m, tiles_n, splits;
+  float beta;
+};
+
+// C = beta C + A B.  One workgroup of NW waves: 16 MT rows of C by 16 NT NW
+// columns, K in steps of 32.
+//   * A is shared by all waves: its fp32 elements come through registers, are
+//     split once and go to LDS as fragments in lane order (lane l = 16 g + r
+//     of a 16-row block holds row r, k = 8g .. 8g+7: 16 bytes per part), so
+//     every LDS write and read is 1 KB in lane order, free of conflicts.  Two
+//     buffers, one barrier per step.
+//   * B's columns belong to one wave each, so B goes straight from global
+//     memory to the registers of the lane that feeds it to the MFMA (lane (n =
+//     l % 16, g): k = 8g .. 8g+7), PD steps ahead, and is split there: no LDS
+//     traffic and no barrier for the operand that is streamed.  B[K,N]: eight
+//     4-byte loads, 16 lanes side by side; B_T: 32 bytes of a row; W4: 4 bytes
+//     of a row and its scale.
+//   * fp32 B: the MFMA takes B first, so a lane ends with 4 consecutive columns
+//     of a row of C.  W4: A first, so a lane's column and scale are one each;
+//     a step is one group of 32 (or part of a longer one), summed from zero and
+//     scaled into the accumulator.
+//   * Nothing depends on the alignment of any operand beyond its type's
+//     (W4: rows of 4-byte aligned bytes).  Rows past M and columns past N read
+//     the last one and are not stored; only the last step reads under a mask.
+//   * What bounds it: large products the MFMA rate the chip sustains (4096^3: 686
+//     us against 1020 for the fp32 MFMA kernel; the MFMA pipe is busy 65% of the
+//     cycles at 1.75 GHz, 1.2 PFLOP/s of bf16, where a bf16 library GEMM reaches
+//     1.1 to 1.4); mid sizes the splitting next to it (128x2048x8192 31.5 us
+//     against 43.0, 301x1537x2003 with B_T 22.8 against 315 for the SIMT kernel
+//     that odd sizes took; a copy without the operand loads runs as long).  W4:
+//     the nibble conversion and the scaling (200x3200x8640: 78 us; one thread
+//     per output took 131 ms).
+//   * A part that overflows or an infinite or NaN operand makes its products
+//     NaN where fp32 arithmetic may give an infinity: tiles with a non-finite
+//     sum are formed again with v_mfma_f32_16x16x4_f32 from the fp32 operands.
+template <int MT, int NT, int NW, int KIND, int PD, int PA = 2>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+    gemm_x3(const X3Args a) {
+  constexpr int CH = (MT + NW - 1) / NW;  // 16-row blocks of A a wave stages
+  constexpr bool W4 = KIND == kBW4;
+  __shared__ uint4 As[2][MT * 3 * 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r16 = lane & 15, g = lane >> 4;
+
+  // XCD-contiguous order over (split, tile): the tiles of one XCD share their
+  // columns of B, or their rows of A, in its L2
+  const int tiles = a.tiles_m * a.tiles_n, nb = tiles * a.splits;
+  int tm, tn, split;
+  {
+    const int q = nb >> 3, r = nb & 7, xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+    const int t = xcd * q + min(xcd, r) + local;
+    split = t / tiles;
+    constexpr int G = 8;
+    const int w = t - split * tiles, gsz = G * a.tiles_n, gi = w / gsz, first = gi * G;
+    const int gm = min(a.tiles_m - first, G), v = w - gi * gsz;
+    tm = first + v % gm;
+    tn = v / gm;
+  }
+  const int m0 = tm * 16 * MT, n0 = (tn * NW + wave) * 16 * NT;
+  const int s0 = split * a.span, s1 = min(s0 + a.span, (a.K + 31) >> 5);
+  const int kend = min(a.K, 32 * s1);
+
+  // ---- operand loads
+  const float *arow[CH];
+#pragma unroll
+  for (int i = 0; i < CH; i++) {
+    const int mt = wave + i * NW;
+    arow[i] = a.A + (int64_t)min(m0 + 16 * mt + r16, a.M - 1) * a.lda + 8 * g;
+  }
+  // a lane's eight floats of a row at step k0 (p is at 8g); `full`: all below K
+  auto load8 = [&](const float *p, int k0, float (&v)[8], auto full) {
+    if constexpr (decltype(full)::value) {
+      const f4u u0 = *(const f4u *)(p + k0), u1 = *(const f4u *)(p + k0 + 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] = u0[e], v[4 + e] = u1[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[e] = k0 + 8 * g + e < a.K ? p[k0 + e] : 0.f;
+    }
+  };
+  struct RawF { float v[NT][8]; };
+  struct RawW { uint32_t w[NT]; float s[NT]; };
+  using Raw = std::conditional_t<W4, RawW, RawF>;
+  const float *brow[NT];    // B_T rows, or the W4 scales
+  const uint8_t *wrow[NT];  // W4 rows
+  uint32_t boff[NT];        // B[K,N]: byte offset of (8g, n)
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+    const int n = min(n0 + 16 * j + r16, a.N - 1);
+    if constexpr (KIND == kBKN) boff[j] = 4u * (uint32_t)(8 * g * (uint32_t)a.ldb + (uint32_t)n);
+    if constexpr (KIND == kBNK) brow[j] = (const float *)a.B + (int64_t)n * a.ldb + 8 * g;
+    if constexpr (W4) {
+      wrow[j] = (const uint8_t *)a.B + (int64_t)n * a.ldb + 4 * g;
+      brow[j] = a.S + (int64_t)n * a.lds;
+    }
+  }
+  const uint32_t ldb4 = 4u * (uint32_t)a.ldb;
+  auto loadb = [&](int s, Raw &r, auto full) {
+    const int k0 = 32 * s;
+    if constexpr (KIND == kBKN) {
+      const char *base = (const char *)a.B + (int64_t)k0 * a.ldb * 4;
+      if constexpr (decltype(full)::value) {
+        // buffer loads: the step's base and the k-row's offset in SGPRs, the
+        // lane's offset fixed, so a load costs no address arithmetic
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 31u * ldb4 + 4u * a.N, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int e = 0; e < 8; e++)
+            r.v[j][e] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(rs, (int)boff[j], (int)(e * ldb4), 0));
+      } else {
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int e = 0; e < 8; e++)
+            r.v[j][e] = k0 + 8 * g + e < a.K
+                            ? *(const float *)(base + (boff[j] + e * ldb4)) : 0.f;
+      }
+    } else if constexpr (KIND == kBNK) {
+#pragma unroll
+      for (int j = 0; j < NT; j++) load8(brow[j], k0, r.v[j], full);
+    } else {
+      const int gr = chunk_group(s, a.cpg, a.cpg_shift);
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        r.w[j] = *(const uint32_t *)(wrow[j] + 16 * s);
+        r.s[j] = brow[j][gr];
+      }
+    }
+  };
+  struct RawA { float v[CH][8]; };
+  auto loada = [&](int s, RawA &r, auto full) {
+#pragma unroll
+    for (int i = 0; i < CH; i++)
+      if (MT % NW == 0 || wave + i * NW < MT) load8(arow[i], 32 * s, r.v[i], full);
+  };
+  auto storea = [&](int buf, const RawA &r) {
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+      const int mt = wave + i * NW;
+      if (MT % NW == 0 || mt < MT) {
+        const Planes p = split8(r.v[i]);
+        As[buf][(mt * 3 + 0) * 64 + lane] = __builtin_bit_cast(uint4, p.h);
+        As[buf][(mt * 3 + 1) * 64 + lane] = __builtin_bit_cast(uint4, p.m);
+        As[buf][(mt * 3 + 2) * 64 + lane] = __builtin_bit_cast(uint4, p.l);
+      }
+    }
+  };
+  // B's fragments of a step: the three parts, or the W4 integers and scales
+  struct FragF { Planes b[NT]; };
+  struct FragW { b8 w[NT]; float s[NT]; };
+  using Frag = std::conditional_t<W4, FragW, FragF>;
+  auto convert = [&](const Raw &r, Frag &f) {
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+      if constexpr (W4) {
+        f.w[j] = nib8_bf16(r.w[j]);
+        f.s[j] = 16.f * r.s[j];
+      } else {
+        f.b[j] = split8(r.v[j]);
+      }
+    }
+  };
+
+  v4f acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  auto frag = [&](int buf, int i) {  // the parts of A's 16-row block i
+    Planes p;
+    p.h = __builtin_bit_cast(b8, As[buf][(i * 3 + 0) * 64 + lane]);
+    p.m = __builtin_bit_cast(b8, As[buf][(i * 3 + 1) * 64 + lane]);
+    p.l = __builtin_bit_cast(b8, As[buf][(i * 3 + 2) * 64 + lane]);
+    return p;
+  };
+  auto compute = [&](int buf, const Frag &f) {
+    if constexpr (W4) {
+#pragma unroll
+      for (int i = 0; i < MT; i++) {
+        const Planes p = frag(buf, i);
+        v4f d[NT];
+#pragma unroll
+        for (int j = 0; j < NT; j++) d[j] = mfma_bf16(p.l, f.w[j], v4f{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int j = 0; j < NT; j++) d[j] = mfma_bf16(p.m, f.w[j], d[j]);
+#pragma unroll
+        for (int j = 0; j < NT; j++) d[j] = mfma_bf16(p.h, f.w[j], d[j]);
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(f.s[j], d[j][e], acc[i][j][e]);
+      }
+    } else {
+      // two row blocks at a time and small parts first: an accumulator's MFMAs
+      // are 2 NT apart
+      constexpr int R = MT % 2 == 0 ? 2 : 1;
+#pragma unroll
+      for (int i = 0; i < MT; i += R) {
+        Planes p[R];
+#pragma unroll
+        for (int q = 0; q < R; q++) p[q] = frag(buf, i + q);
+        auto mul = [&](b8 Planes::*x, b8 Planes::*y) {
+#pragma unroll
+          for (int q = 0; q < R; q++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+              acc[i + q][j] = mfma_bf16(f.b[j].*x, p[q].*y, acc[i + q][j]);
+        };
+        mul(&Planes::h, &Planes::l);
+        mul(&Planes::l, &Planes::h);
+        mul(&Planes::m, &Planes::m);
+        mul(&Planes::h, &Planes::m);
+        mul(&Planes::m, &Planes::h);
+        mul(&Planes::h, &Planes::h);
+      }
+    }
+  };
+
+  // Whole steps s0 .. sf-1, software-pipelined: step s's MFMAs run while step
+  // s+1's operands are split (A into the other LDS buffer, B into registers)
+  // and the loads of the steps up to s+1+PA (A) and s+1+PD (B) are in flight.
+  // Loads return in order, so each step requests its A before its B: waiting
+  // for A then leaves the younger loads of B outstanding.  Loads past the last
+  // whole step repeat it: in bounds, never used.
+  using Full = std::true_type;
+  using Part = std::false_type;
+  const int sf = min(s1, a.K >> 5), last = sf - 1;
+  if (s0 < sf) {
+    RawA ra[PA];
+    Raw rb[PD];
+    Frag fr[2];
+    loada(s0, ra[0], Full{});
+    loadb(s0, rb[0], Full{});
+    storea(0, ra[0]);
+    convert(rb[0], fr[0]);
+#pragma unroll
+    for (int p = 0; p < PA || p < PD; p++) {
+      if (p < PA) loada(min(s0 + 1 + p, last), ra[p], Full{});
+      if (p < PD) loadb(min(s0 + 1 + p, last), rb[p], Full{});
+    }
+    lds_barrier();
+    constexpr int U = PD % 2 == 0 ? PD : 2 * PD;
+    static_assert(U % PA == 0, "unroll");
+    for (int s = s0; s < sf; s += U) {
+#pragma unroll
+      for (int p = 0; p < U; p++) {
+        if (s + p < sf) {  // uniform
+          storea((p & 1) ^ 1, ra[p % PA]);
+          loada(min(s + p + 1 + PA, last), ra[p % PA], Full{});
+          convert(rb[p % PD], fr[(p + 1) & 1]);
+          loadb(min(s + p + 1 + PD, last), rb[p % PD], Full{});
+          compute(p & 1, fr[p & 1]);
+          lds_barrier();
+        }
+      }
+    }
+  }
+  if (sf < s1) {  // the last K % 32 (never for W4)
+    RawA ra;
+    Raw r;
+    Frag f;
+    loada(sf, ra, Part{});
+    loadb(sf, r, Part{});
+    convert(r, f);
+    storea(0, ra);  // the pipeline's last step ended in a barrier
+    lds_barrier();
+    compute(0, f);
+  }
+
+  // ---- scale back; sums that are not finite, again in fp32
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[i][j][e] *= W4 ? 1.f / kUp : 1.f / kUp / kUp;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) bad |= !(fabsf(acc[i][j][e]) <= 3.4028235e38f);
+  if (__builtin_expect(__any(bad), 0)) {
+#pragma unroll 1
+    for (int t = 0; t < MT * NT; t++) {
+      const int ti = t / NT, tj = t - ti * NT;
+      const float *ap = a.A + (int64_t)min(m0 + 16 * ti + r16, a.M - 1) * a.lda;
+      const int n = min(n0 + 16 * tj + r16, a.N - 1);
+      v4f c = {0.f, 0.f, 0.f, 0.f};
+      for (int k = 32 * s0; k < kend; k += 4) {
+        const int kk = k + g;
+        float av = 0.f, bv = 0.f;
+        if (kk < kend) {
+          av = ap[kk];
+          if constexpr (KIND == kBKN) bv = ((const float *)a.B)[(int64_t)kk * a.ldb + n];
+          if constexpr (KIND == kBNK) bv = ((const float *)a.B)[(int64_t)n * a.ldb + kk];
+          if constexpr (W4) {
+            const uint8_t b = ((const uint8_t *)a.B)[(int64_t)n * a.ldb + (kk >> 1)];
+            const int q = (int)((uint32_t)b << (kk & 1 ? 24 : 28)) >> 28;
+            bv = (float)q * a.S[(int64_t)n * a.lds + chunk_group(kk >> 5, a.cpg, a.cpg_shift)];
+          }
+        }
+        c = W4 ? __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, c, 0, 0, 0)
+               : __builtin_amdgcn_mfma_f32_16x16x4f32(bv, av, c, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          if (i * NT + j == t) acc[i][j] = c;
+    }
+  }
+
+  // ---- store
+  float *out = a.P ? a.P + (int64_t)split * a.M * a.N : a.C;
+  const int64_t ldo = a.P ? a.N : a.ldc;
+  const bool add = !a.P && a.beta != 0.f;
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+      if constexpr (W4) {
+        // rows 4g .. 4g+3 of column r16
+        const int n = n0 + 16 * j + r16;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int m = m0 + 16 * i + 4 * g + e;
+          if (m < a.M && n < a.N) {
+            float *o = out + (int64_t)m * ldo + n;
+            *o = add ? *o + acc[i][j][e] : acc[i][j][e];
+          }
+        }
+      } else {
+        // columns 4g .. 4g+3 of row r16
+        const int m = m0 + 16 * i + r16, n = n0 + 16 * j + 4 * g;
+        if (m < a.M) {
+          float *o = out + (int64_t)m * ldo + n;
+          if (n + 3 < a.N) {
+            f4u v = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            if (add) v += *(const f4u *)o;
+            *(f4u *)o = v;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              if (n + e < a.N) o[e] = add ? o[e] + acc[i][j][e] : acc[i][j][e];
+          }
+        }
+      }
+    }
+}
+
+// out[m][n] = beta out + sum over parts p (in order: deterministic) of
+// P[p][m][n]; the loads of B parts are issued together.
+template <int B>
+__global__ void __launch_bounds__(256)
+    x3_sum_parts(const float *__restrict__ P, int parts, float *__restrict__ C, int64_t ldc, int M,
+                 int N, float beta) {
+  const int64_t mn = (int64_t)M * N, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= mn) return;
+  float v = 0.f;
+  for (int s = 0; s < parts; s += B) {
+    float t[B];
+#pragma unroll
+    for (int u = 0; u < B; u++) t[u] = s + u < parts ? P[(int64_t)(s + u) * mn + i] : 0.f;
+#pragma unroll
+    for (int u = 0; u < B; u++)
+      if (s + u < parts) v += t[u];
+  }
+  const int64_t m = i / N;
+  float *o = C + m * ldc + (i - m * N);
+  *o = beta != 0.f ? *o + v : v;
+}
+
+// K splits for `tiles` tiles of `steps` K steps: a round of workgroups over the
+// CUs costs its steps and about four more to fill and drain its pipeline; the
+// partial sums cost a launch (about three steps' time) and their traffic (a
+// step is about 1 us, in which 4 MB go by).  Measured (W4, 200 x 3200 -> 8640,
+// 136 tiles: 1 / 3 / 4 / 6 splits 120 / 77 / 90 / 87 us; fp32 128 x 2048 x 8192,
+// 128 tiles: 1 / 2 / 4 splits 70 / 39 / 39 us).
+int pick_splits(int64_t tiles, int steps, int64_t mn, int64_t cus) {
+  int best = 1;
+  double cost = 0;
+  for (int s = 1; s <= 16 && s * 4 <= std::max(steps, 4); s++) {
+    const int span = (int)cdiv(steps, s);
+    if (cdiv(steps, span) != s) continue;
+    if (s > 1 && s * mn > (int64_t(1) << 28)) break;  // 1 GiB of partials
+    const double c = (double)cdiv(tiles * s, cus) * (span + 4) +
+                     (s > 1 ? 3.0 + 1e-6 * (double)(s + 1) * (double)mn : 0.0);
+    if (s == 1 || c < cost) best = s, cost = c;
+  }
+  return best;
+}
+
+template <int MT, int NT, int NW, int KIND, int PD>
+int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
+  const int64_t cus = num_cus(), tm = cdiv(a.M, 16 * MT), tn = cdiv(a.N, 16 * NT * NW);
+  const int steps = (int)cdiv(a.K, 32);
+  int splits = pick_splits(tm * tn, steps, (int64_t)a.M * a.N, cus);
+  a.P = nullptr;
+  if (splits > 1) {
+    if (may_split && workspace(st, sizeof(float) * (size_t)splits * a.M * a.N, (void **)&a.P, 3) != SIMP_RT_OK) {
+      clear_error();
+      may_split = false;
+    }
+    if (!may_split) {
+      if (!must) return 1;
+      splits = 1;
+      a.P = nullptr;
+    }
+  }
+  a.span = (int)cdiv(steps, splits);
+  a.splits = (int)cdiv(steps, a.span);
+  if (tm * tn * a.splits > INT32_MAX) return 1;
+  a.tiles_m = (int)tm;
+  a.tiles_n = (int)tn;
+  KernelTimer kt(st, "gemm_x3");
+  hipLaunchKernelGGL((gemm_x3<MT, NT, NW, KIND, PD>), dim3((unsigned)(tm * tn * a.splits)),
+                     dim3(64 * NW), 0, st, a);
+  SIMP_HIP(hipGetLastError());
+  if (a.P) {
+    const dim3 g((unsigned)cdiv((int64_t)a.M * a.N, 256));
+    if (a.splits <= 4)
+      hipLaunchKernelGGL(x3_sum_parts<4>, g, dim3(256), 0, st, a.P, a.splits, a.C, a.ldc, a.M, a.N, a.beta);
+    else if (a.splits <= 8)
+      hipLaunchKernelGGL(x3_sum_parts<8>, g, dim3(256), 0, st, a.P, a.splits, a.C, a.ldc, a.M, a.N, a.beta);
+    else
+      hipLaunchKernelGGL(x3_sum_parts<16>, g, dim3(256), 0, st, a.P, a.splits, a.C, a.ldc, a.M, a.N, a.beta);
+    SIMP_HIP(hipGetLastError());
+  }
+  return SIMP_RT_OK;
+}
+
+// Partial sums need the stream's workspace.  A captured call keeps to what it
+// can do without one: a graph must not hold a buffer that a later, larger call
+// may replace.
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
+
+}  // namespace
+
+int launch_x3_f32(bool bt, const float *A, int64_t lda, const float *B, int64_t ldb, float *C,
+                  int64_t ldc, int M, int N, int K, float beta, bool must, hipStream_t st) {
+  // lane and row offsets of B[K,N] are 32-bit: 32 rows within 2 GiB
+  if (M <= 0 || N <= 0 || K <= 0 || (!bt && ldb >= (int64_t(1) << 24))) return 1;
+  X3Args a{};
+  a.A = A;
+  a.lda = lda;
+  a.B = B;
+  a.ldb = ldb;
+  a.C = C;
+  a.ldc = ldc;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.beta = beta;
+  const bool split = !capturing(st);
+  // 16- and 32-row tiles for few rows (24x2048x8192: 16 us on 32x128 tiles of 8
+  // waves, 22 on 32x64 of 4, 20 on 64x128)
+  if (M <= 16)
+    return bt ? go_x3<1, 1, 4, kBNK, 4>(a, split, must, st) : go_x3<1, 1, 4, kBKN, 4>(a, split, must, st);
+  if (M <= 32)
+    return bt ? go_x3<2, 1, 8, kBNK, 4>(a, split, must, st) : go_x3<2, 1, 8, kBKN, 4>(a, split, must, st);
+  // 128x256 tiles from two per CU on (4096^3: 686 us against 790 with 64x128)
+  if (cdiv(M, 128) * cdiv(N, 256) >= 2 * num_cus())
+    return bt ? go_x3<8, 2, 8, kBNK, 2>(a, split, must, st) : go_x3<8, 2, 8, kBKN, 2>(a, split, must, st);
+  return bt ? go_x3<4, 1, 8, kBNK, 4>(a, split, must, st) : go_x3<4, 1, 8, kBKN, 4>(a, split, must, st);
+}
+
+int launch_x3_w4(const uint8_t *W, int64_t ldw, const float *S, int64_t lds, const float *X,
+                 int64_t ldx, float *O, int64_t ldo, int M, int N, int K, int gs, hipStream_t st) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 32 != 0 || gs % 32 != 0 || K % gs != 0 || ldw % 4 != 0 ||
+      ((uintptr_t)W & 3) != 0)
+    return 1;
+  X3Args a{};
+  a.A = X;
+  a.lda = ldx;
+  a.B = W;
+  a.ldb = ldw;
+  a.S = S;
+  a.lds = lds;
+  a.cpg = gs / 32;
+  a.cpg_shift = (a.cpg & (a.cpg - 1)) == 0 ? __builtin_ctz((unsigned)a.cpg) : -1;
+  a.C = O;
+  a.ldc = ldo;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  const bool split = !capturing(st);
+  if (M <= 16) return go_x3<1, 2, 4, kBW4, 4>(a, split, true, st);
+  if (M <= 32) return go_x3<2, 2, 4, kBW4, 4>(a, split, true, st);
+  if (M <= 64) return go_x3<4, 2, 4, kBW4, 4>(a, split, true, st);
+  return go_x3<8, 2, 4, kBW4, 4>(a, split, true, st);
+}
+
+}  // namespace simp

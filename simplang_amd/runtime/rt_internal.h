@@ -204,6 +204,15 @@ struct W4D8Args {
 // K a multiple of 32 and of gs (a multiple of 32), K <= 20480, x0 and nw 16-byte aligned.
 bool w4d8_supported(int K, int gs, const void *x0, const void *nw);
 int launch_w4d8(const W4D8Args &a, hipStream_t st);
+// fp32 and W4 products on the bf16 matrix cores (gemm_x3.hip): C = beta C + A B
+// with B[K,N], or B_T[N,K] (bt); O = X W^T with symmetric W4 rows.  Any
+// alignment and leading dimension; W4: K and gs multiples of 32, rows of W
+// 4-byte aligned.  Return 1 when they do not serve the shape, and (fp32, not
+// `must`) when it wants K splits and their workspace cannot be had.
+int launch_x3_f32(bool bt, const float *A, int64_t lda, const float *B, int64_t ldb, float *C,
+                  int64_t ldc, int M, int N, int K, float beta, bool must, hipStream_t st);
+int launch_x3_w4(const uint8_t *W, int64_t ldw, const float *S, int64_t lds, const float *X,
+                 int64_t ldx, float *O, int64_t ldo, int M, int N, int K, int gs, hipStream_t st);
 // C = beta*C + A*B (beta 0 or 1), row-major with leading dimensions in elements.
 int launch_matmul_f32(const float *A, int64_t lda, const float *B, int64_t ldb, float *C,
                       int64_t ldc, int M, int N, int K, float beta, hipStream_t st);
