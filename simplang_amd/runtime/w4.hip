@@ -605,6 +605,14 @@ int launch_w4s(const uint8_t *W, int64_t ldw, const float *S, int64_t lds, const
   const bool fast = K % 32 == 0 && gs % 32 == 0 && K % gs == 0 && ldw % 16 == 0 &&
                     ((uintptr_t)W & 15) == 0 && ldx % 4 == 0 && ((uintptr_t)X & 15) == 0 &&
                     M <= 16;
+  // groups of more than 32 from five rows of x on: w4s_gemv unpacks to fp32 for
+  // each row (16 x 3200 -> 8640 with groups of 64: 89 us against 20), ahead
+  // only where a launch of its own is all the call costs (8 x 768 x 768: 7.9
+  // against 10.5)
+  if (!fast || (gs != 32 && M >= 5 && (int64_t)M * K * N > (1 << 25))) {
+    const int rc = launch_x3_w4(W, ldw, S, lds, X, ldx, O, ldo, M, N, K, gs, st);
+    if (rc != 1) return rc;
+  }
   if (!fast) {
     const int64_t tot = (int64_t)M * N;
     hipLaunchKernelGGL(w4s_generic, dim3((unsigned)cdiv(tot, 256)), dim3(256), 0, st, W, ldw, S,

@@ -102,3 +102,51 @@ def test_f32_non_finite(dev, nt):
     with np.errstate(invalid="ignore"):
         lim = _bound(K) * (np.abs(a).astype(np.float64) @ np.abs(b))[fin]
     assert (np.abs(got[fin] - want[fin]) <= lim).all()
+
+
+W4 = [(1, 70, 32, 32, 4), (2, 129, 96, 32, 4), (5, 300, 288, 96, 4), (16, 127, 256, 64, 4), (17, 128, 64, 64, 0),
+      (33, 257, 160, 32, 0), (65, 100, 2048, 128, 0), (129, 1, 96, 32, 0), (200, 8640, 320, 64, 0),
+      (8, 1100, 4096, 128, 0)]
+
+
+@pytest.mark.parametrize("M,N,K,gs,pad", W4)
+def test_w4_edges(dev, M, N, K, gs, pad):
+    """pad 4: rows of W that are only 4-byte aligned."""
+    import torch
+    rng = np.random.default_rng(M + N + K)
+    w = rng.integers(0, 256, (N, K // 2 + pad)).astype(np.uint8)
+    s = np.abs(rng.standard_normal((N, K // gs + 1))).astype(np.float32)
+    x = rng.standard_normal((M, K + 1)).astype(np.float32)
+    c = torch.full((M + 1, N + 2), 7.0, device=dev)
+    out = c[:M, 1:N + 1]
+    sa.matmul_w4s(torch.from_numpy(w).to(dev)[:, pad:], torch.from_numpy(s).to(dev)[:, 1:],
+                  torch.from_numpy(x).to(dev)[:, 1:], out, gs)
+    q = w[:, pad:]
+    wd = np.stack([(q << 4).view(np.int8) >> 4, q.view(np.int8) >> 4], -1).reshape(N, K)
+    wd = (wd.reshape(N, -1, gs) * s[:, 1:, None].astype(np.float64)).reshape(N, K)
+    _check(out.cpu().numpy(), x[:, 1:].astype(np.float64), wd.T)
+    full = c.cpu().numpy()
+    assert (full[M] == 7).all() and (full[:, 0] == 7).all() and (full[:, N + 1:] == 7).all()
+
+
+def test_w4_non_finite(dev):
+    import torch
+    rng = np.random.default_rng(9)
+    M, N, K = 40, 200, 128
+    w = rng.integers(0, 256, (N, K // 2)).astype(np.uint8)
+    w[5] = 0x11  # no zero weight in this row
+    s = np.ones((N, K // 32), np.float32)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[0, 3], x[20, 64], x[39, 127] = np.inf, np.nan, -np.inf
+    c = torch.empty(M, N, device=dev)
+    sa.matmul_w4s(torch.from_numpy(w).to(dev), torch.from_numpy(s).to(dev),
+                  torch.from_numpy(x).to(dev), c, 32)
+    wd = np.stack([(w << 4).view(np.int8) >> 4, w.view(np.int8) >> 4], -1).reshape(N, K)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ wd.T.astype(np.float64)
+    got = c.cpu().numpy()
+    fin = np.isfinite(want)
+    assert got[0, 5] == np.inf and np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    lim = _bound(K) * (np.abs(x[1]).astype(np.float64) @ np.abs(wd.T))
+    assert (np.abs(got[1] - want[1]) <= lim).all()
