@@ -591,7 +591,11 @@ int dispatch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, i
   const int64_t kn = (int64_t)K * N;
   const bool small = M <= 32 ? kn < (1 << 20) : BT && M <= 128 && kn <= (5 << 18);
   if (batch == 1 && M > 16 && !one_round && !small) {
-    const int rc = launch_x3_f32(BT, A, lda, B, ldb, C, ldc, M, N, K, beta, false, st);
+    const X3Mat b{B, nullptr, N};
+    // carried sums where the ring kernel would carry its own through all of K;
+    // the smaller shapes, whose K it splits for, keep the closer ones
+    const int rc = launch_x3(&b, 1, ldb, BT ? X3Fmt::kT : X3Fmt::kN, 0, 0, A, lda, C, ldc, M, K,
+                             beta, false, K % 32 == 0 && t64 >= cus, st);
     if (rc != 1) return rc;
   }
   if (M <= 16)
@@ -648,7 +652,9 @@ int launch_gemm_t(const T *A, int64_t lda, int64_t sa, const T *B, int64_t ldb, 
   }
   if constexpr (std::is_same<T, float>::value) {
     if (batch == 1) {
-      const int rc = launch_x3_f32(BT, A, lda, B, ldb, C, ldc, M, N, K, beta, true, st);
+      const X3Mat b{B, nullptr, N};
+      const int rc = launch_x3(&b, 1, ldb, BT ? X3Fmt::kT : X3Fmt::kN, 0, 0, A, lda, C, ldc, M, K,
+                               beta, true, true, st);
       if (rc != 1) return rc;
     }
   }

@@ -44,12 +44,12 @@ struct Planes {
 // in fp32.
 constexpr float kUp = 16777216.f;
 
-// The three bf16 parts of eight floats, scaled by kUp.
-__device__ __forceinline__ Planes split8(const float (&x)[8]) {
+// The three bf16 parts of eight floats, scaled by `up`.
+__device__ __forceinline__ Planes split8(const float (&x)[8], float up = kUp) {
   uint32_t h[4], m[4], l[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const float x0 = kUp * x[2 * i], x1 = kUp * x[2 * i + 1];
+    const float x0 = up * x[2 * i], x1 = up * x[2 * i + 1];
     h[i] = pk_bf16(x0, x1);
     const float r0 = x0 - __uint_as_float(h[i] << 16), r1 = x1 - __uint_as_float(h[i] & 0xFFFF0000u);
     m[i] = pk_bf16(r0, r1);
@@ -81,18 +81,25 @@ __device__ __forceinline__ v4f mfma_bf16(b8 a, b8 b, v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// One of up to three matrices B whose columns stand side by side in C.
+struct X3Part {
+  const void *B;
+  const float *S;    // W4 scales [n, lds], one per `cpg` groups of 32
+  int n;             // columns
+  int c0, t0;        // first column of C, first column tile
+};
 struct X3Args {
   const float *A;
   int64_t lda;
-  const void *B;
+  X3Part part[3];
+  int parts;
   int64_t ldb;       // floats; bytes for W4
-  const float *S;    // W4 scales [N, lds], one per `cpg` groups of 32
   int64_t lds;
   int cpg, cpg_shift;
   float *C;
   int64_t ldc;
   float *P;          // partial products [split][M][N]; null: straight to C
-  int M, N, K;
+  int M, N, K;       // N: the columns of all parts
   int span;          // K steps of 32 per split
   int tiles_m, tiles_n, splits;
   float beta;
@@ -113,8 +120,15 @@ struct X3Args {
 //     of a row and its scale.
 //   * fp32 B: the MFMA takes B first, so a lane ends with 4 consecutive columns
 //     of a row of C.  W4: A first, so a lane's column and scale are one each;
-//     a step is one group of 32 (or part of a longer one), summed from zero and
-//     scaled into the accumulator.
+//     a step is one group of 32 or part of a longer one.
+//   * The bf16 MFMA rounds its sums down (measured: the mean error is half the
+//     root mean square one and negative), so a sum carried through it gathers a
+//     bias that averages over rows do not take out.  So each step is summed
+//     from zero and added to the accumulator by the VALU, which rounds to
+//     nearest, and A's sign turns with every step: 512x4096x4096 is 2e-7 off
+//     64-bit sums (the fp32 MFMA kernel 1.2e-6).  CARRY leaves the sums in the
+//     MFMA accumulator and turns its sign and A's every four steps (1e-6 off;
+//     1024x4096x4096 188 us against 219, 4096^3 690 against 830).
 //   * Nothing depends on the alignment of any operand beyond its type's
 //     (W4: rows of 4-byte aligned bytes).  Rows past M and columns past N read
 //     the last one and are not stored; only the last step reads under a mask.
@@ -129,7 +143,7 @@ struct X3Args {
 //   * A part that overflows or an infinite or NaN operand makes its products
 //     NaN where fp32 arithmetic may give an infinity: tiles with a non-finite
 //     sum are formed again with v_mfma_f32_16x16x4_f32 from the fp32 operands.
-template <int MT, int NT, int NW, int KIND, int PD, int PA = 2>
+template <int MT, int NT, int NW, int KIND, int PD, bool CARRY = false, int PA = 2>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
     gemm_x3(const X3Args a) {
   constexpr int CH = (MT + NW - 1) / NW;  // 16-row blocks of A a wave stages
@@ -152,7 +166,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     tm = first + v % gm;
     tn = v / gm;
   }
-  const int m0 = tm * 16 * MT, n0 = (tn * NW + wave) * 16 * NT;
+  const X3Part b = a.part[(a.parts > 1 && tn >= a.part[1].t0) + (a.parts > 2 && tn >= a.part[2].t0)];
+  const int m0 = tm * 16 * MT, n0 = ((tn - b.t0) * NW + wave) * 16 * NT;
   const int s0 = split * a.span, s1 = min(s0 + a.span, (a.K + 31) >> 5);
   const int kend = min(a.K, 32 * s1);
 
@@ -182,24 +197,24 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
   uint32_t boff[NT];        // B[K,N]: byte offset of (8g, n)
 #pragma unroll
   for (int j = 0; j < NT; j++) {
-    const int n = min(n0 + 16 * j + r16, a.N - 1);
+    const int n = min(n0 + 16 * j + r16, b.n - 1);
     if constexpr (KIND == kBKN) boff[j] = 4u * (uint32_t)(8 * g * (uint32_t)a.ldb + (uint32_t)n);
-    if constexpr (KIND == kBNK) brow[j] = (const float *)a.B + (int64_t)n * a.ldb + 8 * g;
+    if constexpr (KIND == kBNK) brow[j] = (const float *)b.B + (int64_t)n * a.ldb + 8 * g;
     if constexpr (W4) {
-      wrow[j] = (const uint8_t *)a.B + (int64_t)n * a.ldb + 4 * g;
-      brow[j] = a.S + (int64_t)n * a.lds;
+      wrow[j] = (const uint8_t *)b.B + (int64_t)n * a.ldb + 4 * g;
+      brow[j] = b.S + (int64_t)n * a.lds;
     }
   }
   const uint32_t ldb4 = 4u * (uint32_t)a.ldb;
   auto loadb = [&](int s, Raw &r, auto full) {
     const int k0 = 32 * s;
     if constexpr (KIND == kBKN) {
-      const char *base = (const char *)a.B + (int64_t)k0 * a.ldb * 4;
+      const char *base = (const char *)b.B + (int64_t)k0 * a.ldb * 4;
       if constexpr (decltype(full)::value) {
         // buffer loads: the step's base and the k-row's offset in SGPRs, the
         // lane's offset fixed, so a load costs no address arithmetic
         const __amdgpu_buffer_rsrc_t rs =
-            __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 31u * ldb4 + 4u * a.N, 0x00020000);
+            __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 31u * ldb4 + 4u * b.n, 0x00020000);
 #pragma unroll
         for (int j = 0; j < NT; j++)
 #pragma unroll
@@ -232,12 +247,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     for (int i = 0; i < CH; i++)
       if (MT % NW == 0 || wave + i * NW < MT) load8(arow[i], 32 * s, r.v[i], full);
   };
-  auto storea = [&](int buf, const RawA &r) {
+  auto storea = [&](int buf, const RawA &r, float sg) {
 #pragma unroll
     for (int i = 0; i < CH; i++) {
       const int mt = wave + i * NW;
       if (MT % NW == 0 || mt < MT) {
-        const Planes p = split8(r.v[i]);
+        const Planes p = split8(r.v[i], sg * kUp);
         As[buf][(mt * 3 + 0) * 64 + lane] = __builtin_bit_cast(uint4, p.h);
         As[buf][(mt * 3 + 1) * 64 + lane] = __builtin_bit_cast(uint4, p.m);
         As[buf][(mt * 3 + 2) * 64 + lane] = __builtin_bit_cast(uint4, p.l);
@@ -273,7 +288,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     p.l = __builtin_bit_cast(b8, As[buf][(i * 3 + 2) * 64 + lane]);
     return p;
   };
-  auto compute = [&](int buf, const Frag &f) {
+  // the sign of A in step s and of the carried sums
+  auto sign = [&](int s) { return CARRY && ((s - s0) >> 2) & 1 ? -1.f : 1.f; };
+  auto compute = [&](int buf, const Frag &f, float sg) {
     if constexpr (W4) {
 #pragma unroll
       for (int i = 0; i < MT; i++) {
@@ -286,12 +303,14 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
         for (int j = 0; j < NT; j++) d[j] = mfma_bf16(p.h, f.w[j], d[j]);
 #pragma unroll
-        for (int j = 0; j < NT; j++)
+        for (int j = 0; j < NT; j++) {
 #pragma unroll
-          for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(f.s[j], d[j][e], acc[i][j][e]);
+          for (int e = 0; e < 4; e++)
+            acc[i][j][e] = fmaf(sg < 0.f ? -f.s[j] : f.s[j], d[j][e], acc[i][j][e]);
+        }
       }
     } else {
-      // two row blocks at a time and small parts first: an accumulator's MFMAs
+      // two row blocks at a time and small parts first: the MFMAs of one sum
       // are 2 NT apart
       constexpr int R = MT % 2 == 0 ? 2 : 1;
 #pragma unroll
@@ -299,20 +318,44 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         Planes p[R];
 #pragma unroll
         for (int q = 0; q < R; q++) p[q] = frag(buf, i + q);
-        auto mul = [&](b8 Planes::*x, b8 Planes::*y) {
+        v4f d[R][NT];
+        auto mul = [&](b8 Planes::*x, b8 Planes::*y, auto zero) {
+#pragma unroll
+          for (int q = 0; q < R; q++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+              v4f &c = CARRY ? acc[i + q][j] : d[q][j];
+              c = mfma_bf16(f.b[j].*x, p[q].*y,
+                            decltype(zero)::value ? v4f{0.f, 0.f, 0.f, 0.f} : c);
+            }
+        };
+        mul(&Planes::h, &Planes::l, std::bool_constant<!CARRY>{});
+        mul(&Planes::l, &Planes::h, std::false_type{});
+        mul(&Planes::m, &Planes::m, std::false_type{});
+        mul(&Planes::h, &Planes::m, std::false_type{});
+        mul(&Planes::m, &Planes::h, std::false_type{});
+        mul(&Planes::h, &Planes::h, std::false_type{});
+        if constexpr (!CARRY) {
 #pragma unroll
           for (int q = 0; q < R; q++)
 #pragma unroll
             for (int j = 0; j < NT; j++)
-              acc[i + q][j] = mfma_bf16(f.b[j].*x, p[q].*y, acc[i + q][j]);
-        };
-        mul(&Planes::h, &Planes::l);
-        mul(&Planes::l, &Planes::h);
-        mul(&Planes::m, &Planes::m);
-        mul(&Planes::h, &Planes::m);
-        mul(&Planes::m, &Planes::h);
-        mul(&Planes::h, &Planes::h);
+#pragma unroll
+              for (int e = 0; e < 4; e++)
+                acc[i + q][j][e] = sg < 0.f ? acc[i + q][j][e] - d[q][j][e]
+                                            : acc[i + q][j][e] + d[q][j][e];
+        }
       }
+    }
+  };
+  auto negate = [&] {
+    if constexpr (CARRY) {
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[i][j][e] = -acc[i][j][e];
     }
   };
 
@@ -325,13 +368,14 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
   using Full = std::true_type;
   using Part = std::false_type;
   const int sf = min(s1, a.K >> 5), last = sf - 1;
+  const int sg0 = s0 + max(sf - s0, 0) / 4 * 4;  // end of the whole runs of four
   if (s0 < sf) {
     RawA ra[PA];
     Raw rb[PD];
     Frag fr[2];
     loada(s0, ra[0], Full{});
     loadb(s0, rb[0], Full{});
-    storea(0, ra[0]);
+    storea(0, ra[0], 1.f);
     convert(rb[0], fr[0]);
 #pragma unroll
     for (int p = 0; p < PA || p < PD; p++) {
@@ -339,19 +383,31 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
       if (p < PD) loadb(min(s0 + 1 + p, last), rb[p], Full{});
     }
     lds_barrier();
-    constexpr int U = PD % 2 == 0 ? PD : 2 * PD;
-    static_assert(U % PA == 0, "unroll");
-    for (int s = s0; s < sf; s += U) {
-#pragma unroll
-      for (int p = 0; p < U; p++) {
-        if (s + p < sf) {  // uniform
-          storea((p & 1) ^ 1, ra[p % PA]);
-          loada(min(s + p + 1 + PA, last), ra[p % PA], Full{});
-          convert(rb[p % PD], fr[(p + 1) & 1]);
-          loadb(min(s + p + 1 + PD, last), rb[p % PD], Full{});
-          compute(p & 1, fr[p & 1]);
-          lds_barrier();
-        }
+    static_assert(4 % PD == 0 && 4 % PA == 0, "unroll");
+    auto step = [&](int s, auto pp) {
+      constexpr int p = decltype(pp)::value;
+      // the sign of A in this step and in the next
+      const float sg = CARRY ? sign(s) : p & 1 ? -1.f : 1.f, sn = CARRY ? sign(s + 1) : -sg;
+      storea((p & 1) ^ 1, ra[p % PA], sn);
+      loada(min(s + 1 + PA, last), ra[p % PA], Full{});
+      convert(rb[p % PD], fr[(p + 1) & 1]);
+      loadb(min(s + 1 + PD, last), rb[p % PD], Full{});
+      compute(p & 1, fr[p & 1], sg);
+      lds_barrier();
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    // (a test before each step keeps the compiler from merging the four: merged,
+    // W4 ran 16% longer and fp32 10%)
+    for (int s = s0; s < sf; s += 4) {
+      step(s, I0{});
+      if (s + 1 < sf) step(s + 1, I1{});
+      if (s + 2 < sf) step(s + 2, I2{});
+      if (s + 3 < sf) {
+        step(s + 3, I3{});
+        negate();
       }
     }
   }
@@ -362,18 +418,19 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     loada(sf, ra, Part{});
     loadb(sf, r, Part{});
     convert(r, f);
-    storea(0, ra);  // the pipeline's last step ended in a barrier
+    storea(0, ra, sign(sg0));  // the pipeline's last step ended in a barrier
     lds_barrier();
-    compute(0, f);
+    compute(0, f, sign(sg0));
   }
 
   // ---- scale back; sums that are not finite, again in fp32
+  const float down = (W4 ? 1.f / kUp : 1.f / kUp / kUp) * (CARRY ? sign(sg0) : 1.f);
 #pragma unroll
   for (int i = 0; i < MT; i++)
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) acc[i][j][e] *= W4 ? 1.f / kUp : 1.f / kUp / kUp;
+      for (int e = 0; e < 4; e++) acc[i][j][e] *= down;
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < MT; i++)
@@ -386,19 +443,19 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     for (int t = 0; t < MT * NT; t++) {
       const int ti = t / NT, tj = t - ti * NT;
       const float *ap = a.A + (int64_t)min(m0 + 16 * ti + r16, a.M - 1) * a.lda;
-      const int n = min(n0 + 16 * tj + r16, a.N - 1);
+      const int n = min(n0 + 16 * tj + r16, b.n - 1);
       v4f c = {0.f, 0.f, 0.f, 0.f};
       for (int k = 32 * s0; k < kend; k += 4) {
         const int kk = k + g;
         float av = 0.f, bv = 0.f;
         if (kk < kend) {
           av = ap[kk];
-          if constexpr (KIND == kBKN) bv = ((const float *)a.B)[(int64_t)kk * a.ldb + n];
-          if constexpr (KIND == kBNK) bv = ((const float *)a.B)[(int64_t)n * a.ldb + kk];
+          if constexpr (KIND == kBKN) bv = ((const float *)b.B)[(int64_t)kk * a.ldb + n];
+          if constexpr (KIND == kBNK) bv = ((const float *)b.B)[(int64_t)n * a.ldb + kk];
           if constexpr (W4) {
-            const uint8_t b = ((const uint8_t *)a.B)[(int64_t)n * a.ldb + (kk >> 1)];
-            const int q = (int)((uint32_t)b << (kk & 1 ? 24 : 28)) >> 28;
-            bv = (float)q * a.S[(int64_t)n * a.lds + chunk_group(kk >> 5, a.cpg, a.cpg_shift)];
+            const uint8_t w = ((const uint8_t *)b.B)[(int64_t)n * a.ldb + (kk >> 1)];
+            const int q = (int)((uint32_t)w << (kk & 1 ? 24 : 28)) >> 28;
+            bv = (float)q * b.S[(int64_t)n * a.lds + chunk_group(kk >> 5, a.cpg, a.cpg_shift)];
           }
         }
         c = W4 ? __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, c, 0, 0, 0)
@@ -413,7 +470,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
   }
 
   // ---- store
-  float *out = a.P ? a.P + (int64_t)split * a.M * a.N : a.C;
+  float *out = (a.P ? a.P + (int64_t)split * a.M * a.N : a.C) + b.c0;
   const int64_t ldo = a.P ? a.N : a.ldc;
   const bool add = !a.P && a.beta != 0.f;
 #pragma unroll
@@ -426,7 +483,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const int m = m0 + 16 * i + 4 * g + e;
-          if (m < a.M && n < a.N) {
+          if (m < a.M && n < b.n) {
             float *o = out + (int64_t)m * ldo + n;
             *o = add ? *o + acc[i][j][e] : acc[i][j][e];
           }
@@ -436,14 +493,14 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
         const int m = m0 + 16 * i + r16, n = n0 + 16 * j + 4 * g;
         if (m < a.M) {
           float *o = out + (int64_t)m * ldo + n;
-          if (n + 3 < a.N) {
+          if (n + 3 < b.n) {
             f4u v = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
             if (add) v += *(const f4u *)o;
             *(f4u *)o = v;
           } else {
 #pragma unroll
             for (int e = 0; e < 4; e++)
-              if (n + e < a.N) o[e] = add ? o[e] + acc[i][j][e] : acc[i][j][e];
+              if (n + e < b.n) o[e] = add ? o[e] + acc[i][j][e] : acc[i][j][e];
           }
         }
       }
@@ -492,9 +549,17 @@ int pick_splits(int64_t tiles, int steps, int64_t mn, int64_t cus) {
   return best;
 }
 
-template <int MT, int NT, int NW, int KIND, int PD>
+template <int MT, int NT, int NW, int KIND, int PD, bool CARRY = false>
 int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
-  const int64_t cus = num_cus(), tm = cdiv(a.M, 16 * MT), tn = cdiv(a.N, 16 * NT * NW);
+  const int64_t cus = num_cus(), tm = cdiv(a.M, 16 * MT);
+  int64_t tn = 0;
+  a.N = 0;
+  for (int i = 0; i < a.parts; i++) {
+    a.part[i].c0 = a.N;
+    a.part[i].t0 = (int)tn;
+    a.N += a.part[i].n;
+    tn += cdiv(a.part[i].n, 16 * NT * NW);
+  }
   const int steps = (int)cdiv(a.K, 32);
   int splits = pick_splits(tm * tn, steps, (int64_t)a.M * a.N, cus);
   a.P = nullptr;
@@ -515,7 +580,7 @@ int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
   a.tiles_m = (int)tm;
   a.tiles_n = (int)tn;
   KernelTimer kt(st, "gemm_x3");
-  hipLaunchKernelGGL((gemm_x3<MT, NT, NW, KIND, PD>), dim3((unsigned)(tm * tn * a.splits)),
+  hipLaunchKernelGGL((gemm_x3<MT, NT, NW, KIND, PD, CARRY>), dim3((unsigned)(tm * tn * a.splits)),
                      dim3(64 * NW), 0, st, a);
   SIMP_HIP(hipGetLastError());
   if (a.P) {
@@ -541,58 +606,53 @@ bool capturing(hipStream_t st) {
 
 }  // namespace
 
-int launch_x3_f32(bool bt, const float *A, int64_t lda, const float *B, int64_t ldb, float *C,
-                  int64_t ldc, int M, int N, int K, float beta, bool must, hipStream_t st) {
+int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, int gs,
+              const float *A, int64_t lda, float *C, int64_t ldc, int M, int K, float beta,
+              bool must, bool carry, hipStream_t st) {
+  int64_t N = 0;
+  for (int i = 0; i < nmat; i++) N += mats[i].n;
+  if (M <= 0 || N <= 0 || N > INT32_MAX || K <= 0 || nmat > 3) return 1;
   // lane and row offsets of B[K,N] are 32-bit: 32 rows within 2 GiB
-  if (M <= 0 || N <= 0 || K <= 0 || (!bt && ldb >= (int64_t(1) << 24))) return 1;
+  if (fmt == X3Fmt::kN && ldb >= (int64_t(1) << 24)) return 1;
   X3Args a{};
+  if (fmt == X3Fmt::kW4) {
+    if (K % 32 != 0 || gs % 32 != 0 || K % gs != 0 || ldb % 4 != 0) return 1;
+    a.cpg = gs / 32;
+    a.cpg_shift = (a.cpg & (a.cpg - 1)) == 0 ? __builtin_ctz((unsigned)a.cpg) : -1;
+  }
+  for (int i = 0; i < nmat; i++) {
+    if (fmt == X3Fmt::kW4 && ((uintptr_t)mats[i].B & 3) != 0) return 1;
+    a.part[i] = X3Part{mats[i].B, mats[i].S, mats[i].n, 0, 0};
+  }
+  a.parts = nmat;
   a.A = A;
   a.lda = lda;
-  a.B = B;
   a.ldb = ldb;
+  a.lds = lds;
   a.C = C;
   a.ldc = ldc;
   a.M = M;
-  a.N = N;
   a.K = K;
   a.beta = beta;
   const bool split = !capturing(st);
+#define X3_GO(MT, NT, NW, ...)                                                         \
+  (fmt == X3Fmt::kN ? go_x3<MT, NT, NW, kBKN, __VA_ARGS__>(a, split, must, st)          \
+                    : go_x3<MT, NT, NW, kBNK, __VA_ARGS__>(a, split, must, st))
+  if (fmt == X3Fmt::kW4) {
+    if (M <= 16) return go_x3<1, 2, 4, kBW4, 4>(a, split, must, st);
+    if (M <= 32) return go_x3<2, 2, 4, kBW4, 4>(a, split, must, st);
+    if (M <= 64) return go_x3<4, 2, 4, kBW4, 4>(a, split, must, st);
+    return go_x3<8, 2, 4, kBW4, 4>(a, split, must, st);
+  }
   // 16- and 32-row tiles for few rows (24x2048x8192: 16 us on 32x128 tiles of 8
   // waves, 22 on 32x64 of 4, 20 on 64x128)
-  if (M <= 16)
-    return bt ? go_x3<1, 1, 4, kBNK, 4>(a, split, must, st) : go_x3<1, 1, 4, kBKN, 4>(a, split, must, st);
-  if (M <= 32)
-    return bt ? go_x3<2, 1, 8, kBNK, 4>(a, split, must, st) : go_x3<2, 1, 8, kBKN, 4>(a, split, must, st);
+  if (M <= 16) return X3_GO(1, 1, 4, 4);
+  if (M <= 32) return X3_GO(2, 1, 8, 4);
   // 128x256 tiles from two per CU on (4096^3: 686 us against 790 with 64x128)
-  if (cdiv(M, 128) * cdiv(N, 256) >= 2 * num_cus())
-    return bt ? go_x3<8, 2, 8, kBNK, 2>(a, split, must, st) : go_x3<8, 2, 8, kBKN, 2>(a, split, must, st);
-  return bt ? go_x3<4, 1, 8, kBNK, 4>(a, split, must, st) : go_x3<4, 1, 8, kBKN, 4>(a, split, must, st);
-}
-
-int launch_x3_w4(const uint8_t *W, int64_t ldw, const float *S, int64_t lds, const float *X,
-                 int64_t ldx, float *O, int64_t ldo, int M, int N, int K, int gs, hipStream_t st) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % 32 != 0 || gs % 32 != 0 || K % gs != 0 || ldw % 4 != 0 ||
-      ((uintptr_t)W & 3) != 0)
-    return 1;
-  X3Args a{};
-  a.A = X;
-  a.lda = ldx;
-  a.B = W;
-  a.ldb = ldw;
-  a.S = S;
-  a.lds = lds;
-  a.cpg = gs / 32;
-  a.cpg_shift = (a.cpg & (a.cpg - 1)) == 0 ? __builtin_ctz((unsigned)a.cpg) : -1;
-  a.C = O;
-  a.ldc = ldo;
-  a.M = M;
-  a.N = N;
-  a.K = K;
-  const bool split = !capturing(st);
-  if (M <= 16) return go_x3<1, 2, 4, kBW4, 4>(a, split, true, st);
-  if (M <= 32) return go_x3<2, 2, 4, kBW4, 4>(a, split, true, st);
-  if (M <= 64) return go_x3<4, 2, 4, kBW4, 4>(a, split, true, st);
-  return go_x3<8, 2, 4, kBW4, 4>(a, split, true, st);
+  if (carry && cdiv(M, 128) * cdiv(N, 256) >= 2 * num_cus()) return X3_GO(8, 2, 8, 2, true);
+  if (carry) return X3_GO(4, 1, 8, 4, true);
+  return X3_GO(4, 1, 8, 4);
+#undef X3_GO
 }
 
 }  // namespace simp

@@ -205,14 +205,39 @@ struct W4D8Args {
 bool w4d8_supported(int K, int gs, const void *x0, const void *nw);
 int launch_w4d8(const W4D8Args &a, hipStream_t st);
 // fp32 and W4 products on the bf16 matrix cores (gemm_x3.hip): C = beta C + A B
-// with B[K,N], or B_T[N,K] (bt); O = X W^T with symmetric W4 rows.  Any
-// alignment and leading dimension; W4: K and gs multiples of 32, rows of W
-// 4-byte aligned.  Return 1 when they do not serve the shape, and (fp32, not
-// `must`) when it wants K splits and their workspace cannot be had.
-int launch_x3_f32(bool bt, const float *A, int64_t lda, const float *B, int64_t ldb, float *C,
-                  int64_t ldc, int M, int N, int K, float beta, bool must, hipStream_t st);
-int launch_x3_w4(const uint8_t *W, int64_t ldw, const float *S, int64_t lds, const float *X,
-                 int64_t ldx, float *O, int64_t ldo, int M, int N, int K, int gs, hipStream_t st);
+// for up to three B whose columns stand side by side in C: B[K,n], B_T[n,K], or
+// symmetric W4 rows [n, K/2] with scales [n, lds].  Any alignment and leading
+// dimension; W4: K and gs multiples of 32, rows of W 4-byte aligned.  Returns 1
+// when it does not serve the shape, and, unless `must`, when it wants K splits
+// and their workspace cannot be had.  `carry` (fp32): sums may be carried
+// through the whole of K in the MFMA accumulator, faster and as exact as the
+// fp32 MFMA kernels' over as long a K; else they are several times more exact.
+enum class X3Fmt { kN, kT, kW4 };
+struct X3Mat {
+  const void *B;
+  const float *S;
+  int n;
+};
+int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, int gs,
+              const float *A, int64_t lda, float *C, int64_t ldc, int M, int K, float beta,
+              bool must, bool carry, hipStream_t st);
+
+// The tokens of a prompt, positions [p0, p0 + T), through all layers of the
+// decode engine at once (prefill.hip): fills the K/V cache rows of those
+// positions, as T steps would.
+struct PrefillArgs {
+  const simp_rt_llama_config *cfg;
+  const simp_rt_llama_weights *w;
+  int kv_dim, hs;
+  const int *prompt;      // device
+  float *kcache, *vcache; // [n_layers, seq_len, kv_dim]
+  const float2 *rope;     // [seq_len, hs / 2], or null
+  float *ws;              // prefill_floats(cfg, rows) floats
+  int rows;               // tokens per pass
+};
+bool prefill_supported(const simp_rt_llama_config &cfg, int hs);
+size_t prefill_floats(const simp_rt_llama_config &cfg, int rows);
+int prefill(const PrefillArgs &a, int64_t n_tokens, hipStream_t st);
 // C = beta*C + A*B (beta 0 or 1), row-major with leading dimensions in elements.
 int launch_matmul_f32(const float *A, int64_t lda, const float *B, int64_t ldb, float *C,
                       int64_t ldc, int M, int N, int K, float beta, hipStream_t st);

@@ -610,7 +610,9 @@ int launch_w4s(const uint8_t *W, int64_t ldw, const float *S, int64_t lds, const
   // only where a launch of its own is all the call costs (8 x 768 x 768: 7.9
   // against 10.5)
   if (!fast || (gs != 32 && M >= 5 && (int64_t)M * K * N > (1 << 25))) {
-    const int rc = launch_x3_w4(W, ldw, S, lds, X, ldx, O, ldo, M, N, K, gs, st);
+    const X3Mat b{W, S, N};
+    const int rc = launch_x3(&b, 1, ldw, X3Fmt::kW4, lds, gs, X, ldx, O, ldo, M, K, 0.f, true, false,
+                             st);
     if (rc != 1) return rc;
   }
   if (!fast) {
