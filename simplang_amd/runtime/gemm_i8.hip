@@ -73,7 +73,32 @@ __device__ __forceinline__ void transpose4x4(uint32_t d0, uint32_t d1, uint32_t 
   o3 = __builtin_amdgcn_perm(y1, x1, 0x07060302u);
 }
 
-template <int BM, int BN, int BK, int WGM, int WGN, bool BNK, bool AU8, bool ATOMIC>
+// Sixteen and four bytes at any address (the type says so; the compiler picks
+// the instructions).
+typedef uint32_t u4any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u1any __attribute__((aligned(1)));
+
+// 16 bytes of a row of K from k on: whole, or, with fewer than 16 left, the last
+// 16 of the row shifted down (zeros above; K >= 16).
+__device__ __forceinline__ uint4 row16_any(const int8_t *row, int k, int K) {
+  if (k + 16 <= K) {
+    const u4any v = *(const u4any *)(row + k);
+    return make_uint4(v.x, v.y, v.z, v.w);
+  }
+  const u4any v = *(const u4any *)(row + K - 16);
+  const int sh = 8 * (k + 16 - K);  // 8 .. 120
+  uint64_t lo = v.x | (uint64_t)v.y << 32, hi = v.z | (uint64_t)v.w << 32;
+  if (sh >= 64) lo = hi >> (sh - 64), hi = 0;
+  else lo = lo >> sh | hi << (64 - sh), hi >>= sh;
+  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+
+// ANY: any K >= 16, leading dimension and alignment (and N >= 4 for B[K,N]):
+// rows end inside a 16-byte chunk and nothing is aligned, so the loads are
+// byte-aligned ones, and a row's last chunk (a k-row's last four columns) is
+// read from where its last 16 (4) bytes start and shifted down.  Bytes of A past
+// K meet zeros of B.
+template <int BM, int BN, int BK, int WGM, int WGN, bool BNK, bool AU8, bool ATOMIC, bool ANY = false>
 __global__ void __launch_bounds__(WGM *WGN * 64)
     gemm_i8_mfma(const int8_t *__restrict__ A, int64_t lda, const int8_t *__restrict__ B,
                  int64_t ldb, int32_t *__restrict__ C, int64_t ldc, int M, int N, int K,
@@ -117,7 +142,8 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
       if (A_TOT % NT == 0 || c < A_TOT) {
         const int kc = c % KC, m = c / KC;
         const int gm = m0 + m, gk = k0 + kc * 16;
-        if (gm < M && gk < kend) v = *(const uint4 *)(A + (int64_t)gm * lda + gk);
+        if (gm < M && gk < kend)
+          v = ANY ? row16_any(A + (int64_t)gm * lda, gk, K) : *(const uint4 *)(A + (int64_t)gm * lda + gk);
       }
       ra[i] = v;
     }
@@ -129,7 +155,8 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
         if (B_TOT % NT == 0 || c < B_TOT) {
           const int kc = c % KC, n = c / KC;
           const int gn = n0 + n, gk = k0 + kc * 16;
-          if (gn < N && gk < kend) v = *(const uint4 *)(B + (int64_t)gn * ldb + gk);
+          if (gn < N && gk < kend)
+            v = ANY ? row16_any(B + (int64_t)gn * ldb, gk, K) : *(const uint4 *)(B + (int64_t)gn * ldb + gk);
         }
         rbq[i] = v;
       }
@@ -140,11 +167,15 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
         const bool on = (B_TOT % NT == 0 || u < B_TOT);
         const int nq = u % (BN / 4), kq = u / (BN / 4);
         const int gn = n0 + nq * 4;
-        const int8_t *p = B + (int64_t)(k0 + kq * 16) * ldb + gn;
+        const int back = ANY ? max(0, min(gn + 4 - N, 3)) : 0;  // columns past N in this group
+        const int8_t *p = B + (int64_t)(k0 + kq * 16) * ldb + gn - back;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int gk = k0 + kq * 16 + r;
-          rbd[i][r] = (on && gn < N && gk < kend) ? *(const uint32_t *)(p + (int64_t)r * ldb) : 0u;
+          rbd[i][r] = 0u;
+          if (on && gn < N && gk < kend)
+            rbd[i][r] = ANY ? *(const u1any *)(p + (int64_t)r * ldb) >> (8 * back)
+                            : *(const uint32_t *)(p + (int64_t)r * ldb);
         }
       }
     }
@@ -1116,7 +1147,7 @@ struct GemmArgs {
   size_t scratch_bytes = 0;
 };
 
-template <int BM, int BN, int BK, int WGM, int WGN, bool BNK, bool AU8>
+template <int BM, int BN, int BK, int WGM, int WGN, bool BNK, bool AU8, bool ANY = false>
 int launch_mfma(const GemmArgs &g, int splits, hipStream_t st) {
   const int tiles_m = (int)cdiv(g.M, BM), tiles_n = (int)cdiv(g.N, BN);
   const int nkt = (int)cdiv(g.K, BK);
@@ -1129,16 +1160,36 @@ int launch_mfma(const GemmArgs &g, int splits, hipStream_t st) {
     const int64_t tot = (int64_t)g.M * g.N;
     hipLaunchKernelGGL(fill_i32_2d, dim3((unsigned)cdiv(tot, 256), 1, g.batch), dim3(256), 0, st,
                        g.C, g.ldc, g.M, g.N, g.sc);
-    hipLaunchKernelGGL((gemm_i8_mfma<BM, BN, BK, WGM, WGN, BNK, AU8, true>), grid, block, 0, st,
+    hipLaunchKernelGGL((gemm_i8_mfma<BM, BN, BK, WGM, WGN, BNK, AU8, true, ANY>), grid, block, 0, st,
                        g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M, g.N, g.K, tiles_m, tiles_n,
                        k_span, g.sa, g.sb, g.sc);
   } else {
-    hipLaunchKernelGGL((gemm_i8_mfma<BM, BN, BK, WGM, WGN, BNK, AU8, false>), grid, block, 0,
+    hipLaunchKernelGGL((gemm_i8_mfma<BM, BN, BK, WGM, WGN, BNK, AU8, false, ANY>), grid, block, 0,
                        st, g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M, g.N, g.K, tiles_m, tiles_n,
                        k_span, g.sa, g.sb, g.sc);
   }
   SIMP_HIP(hipGetLastError());
   return SIMP_RT_OK;
+}
+
+// Register-staged tiles by size.
+template <bool BNK, bool AU8, bool ANY>
+int dispatch_tiles(const GemmArgs &g, hipStream_t st) {
+  const int64_t cus = num_cus();
+  auto tiles = [&](int bm, int bn) { return cdiv(g.M, bm) * cdiv(g.N, bn); };
+  // Split K for about four workgroups per CU (at most 16 splits): 8x8640x3200
+  // 9.4 us with 8 splits against 12.5 with the 4 that two per CU gave and 10.7
+  // with 16; the 768 / 2048 shapes reach their K or the cap either way.  One
+  // split (no zero fill, no atomics) is 1.6-3.5x slower at these sizes.
+  if (tiles(128, 128) * g.batch >= cus) return launch_mfma<128, 128, 128, 2, 2, BNK, AU8, ANY>(g, 1, st);
+  if (g.M > 32) {
+    const int64_t t = tiles(64, 64) * g.batch;
+    const int s = (int)std::min<int64_t>(cdiv(4 * cus, t), 16);
+    return launch_mfma<64, 64, 128, 2, 2, BNK, AU8, ANY>(g, t >= cus ? 1 : s, st);
+  }
+  const int64_t t = tiles(32, 64) * g.batch;
+  const int s = (int)std::min<int64_t>(cdiv(4 * cus, t), 16);
+  return launch_mfma<32, 64, 128, 1, 2, BNK, AU8, ANY>(g, t >= cus ? 1 : s, st);
 }
 
 template <bool BNK, bool AU8>
@@ -1172,6 +1223,8 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
   const bool b_ok = BNK ? (g.ldb % 16 == 0 && ((uintptr_t)g.B & 15) == 0 && g.sb % 16 == 0)
                         : (g.N % 4 == 0 && g.ldb % 4 == 0 && ((uintptr_t)g.B & 3) == 0 &&
                            g.sb % 4 == 0);
+  if ((!a_ok || !b_ok) && g.K >= 16 && (BNK || g.N >= 4))
+    return dispatch_tiles<BNK, AU8, true>(g, st);
   if (!a_ok || !b_ok) {
     dim3 grid((unsigned)cdiv(g.N, 64), (unsigned)std::min<int64_t>(cdiv(g.M, 4), 65535),
               g.batch);
@@ -1353,19 +1406,7 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
       return SIMP_RT_OK;
     }
   }
-  // Split K for about four workgroups per CU (at most 16 splits): 8x8640x3200
-  // 9.4 us with 8 splits against 12.5 with the 4 that two per CU gave and 10.7
-  // with 16; the 768 / 2048 shapes reach their K or the cap either way.  One
-  // split (no zero fill, no atomics) is 1.6-3.5x slower at these sizes.
-  if (tiles(128, 128) * g.batch >= cus) return launch_mfma<128, 128, 128, 2, 2, BNK, AU8>(g, 1, st);
-  if (g.M > 32) {
-    const int64_t t = tiles(64, 64) * g.batch;
-    const int s = (int)std::min<int64_t>(cdiv(4 * cus, t), 16);
-    return launch_mfma<64, 64, 128, 2, 2, BNK, AU8>(g, t >= cus ? 1 : s, st);
-  }
-  const int64_t t = tiles(32, 64) * g.batch;
-  const int s = (int)std::min<int64_t>(cdiv(4 * cus, t), 16);
-  return launch_mfma<32, 64, 128, 1, 2, BNK, AU8>(g, t >= cus ? 1 : s, st);
+  return dispatch_tiles<BNK, AU8, false>(g, st);
 }
 
 // ------------------------------------------------------------------ int4 --

@@ -1,0 +1,48 @@
+"""int8 products whose sizes, leading dimensions or bases are not multiples of 16
+bytes: exact against float64 products (sums below 2^53)."""
+import numpy as np
+import pytest
+
+import simplang_amd as sa
+
+pytestmark = pytest.mark.gpu
+
+# K around 16, 32 and the 128-deep step, with remainders; N % 4 of 0 to 3, below
+# and above a tile; one and several K splits; 128x128 tiles (2049x2055)
+SHAPES = [(1, 5, 17), (2, 3, 40), (3, 4, 16), (5, 6, 15), (33, 67, 31), (40, 64, 129), (64, 131, 255),
+          (100, 258, 1533), (7, 4099, 1025), (2049, 2055, 100), (129, 130, 143)]
+
+
+@pytest.mark.parametrize("u8", [False, True])
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_any_size_and_alignment(dev, M, N, K, nt, u8):
+    import torch
+    rng = np.random.default_rng(M + 3 * N + 5 * K)
+    lo, dt = (0, np.uint8) if u8 else (-128, np.int8)
+    a = rng.integers(lo, lo + 256, (M, K)).astype(dt)
+    b = rng.integers(-128, 128, (N, K) if nt else (K, N)).astype(np.int8)
+    fn = {(False, False): sa.tensor_matmul_i8, (False, True): sa.matmul_u8s8_i32,
+          (True, False): sa.tensor_matmul_nt_i8, (True, True): sa.matmul_nt_u8s8_i32}[nt, u8]
+    want = (a.astype(np.float64) @ (b.T if nt else b).astype(np.float64)).astype(np.int64)
+    # dense (the last rows end with the allocation), and views with odd pitches
+    for off, pad in ((0, 0), (1, 2), (3, 13)):
+        at = torch.zeros(M, K + off + pad, dtype=torch.uint8 if u8 else torch.int8)
+        bt = torch.full((b.shape[0], b.shape[1] + off + pad), 77, dtype=torch.int8)
+        at[:, off:off + K] = torch.from_numpy(a)
+        bt[:, off:off + b.shape[1]] = torch.from_numpy(b)
+        c = torch.full((M + 1, N + 1), 9, dtype=torch.int32, device=dev)
+        fn(at.to(dev)[:, off:off + K], bt.to(dev)[:, off:off + b.shape[1]], c[:M, :N])
+        got = c.cpu().numpy()
+        assert np.array_equal(got[:M, :N], want), (off, pad)
+        assert (got[M] == 9).all() and (got[:, N] == 9).all()
+
+
+def test_any_batch(dev):
+    import torch
+    rng = np.random.default_rng(1)
+    a = rng.integers(-128, 128, (5, 37, 83)).astype(np.int8)
+    b = rng.integers(-128, 128, (5, 83, 45)).astype(np.int8)
+    c = torch.empty(5, 37, 45, dtype=torch.int32, device=dev)
+    sa.tensor_batch_matmul(torch.from_numpy(a).to(dev), torch.from_numpy(b).to(dev), c)
+    assert np.array_equal(c.cpu().numpy(), (a.astype(np.float64) @ b.astype(np.float64)).astype(np.int32))
