@@ -77,6 +77,8 @@ __device__ __forceinline__ void transpose4x4(uint32_t d0, uint32_t d1, uint32_t 
 // the instructions).
 typedef uint32_t u4any __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t u1any __attribute__((aligned(1)));
+// Four i32 of a row of C that is only 4-byte aligned.
+typedef int v4i_u __attribute__((ext_vector_type(4), aligned(4)));
 
 // 16 bytes of a row of K from k on: whole, or, with fewer than 16 left, the last
 // 16 of the row shifted down (zeros above; K >= 16).
@@ -674,6 +676,8 @@ __global__ void __launch_bounds__(512)
           // at a tile's end drains faster without allocating in L2 (measured
           // 4-5% on the whole kernel at 8192^3)
           __builtin_nontemporal_store(v, (v4i *)dst);
+        } else if (col + 3 < N) {
+          *(v4i_u *)dst = v;
         } else {
 #pragma unroll
           for (int r = 0; r < 4; r++)
@@ -908,6 +912,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN)
         int32_t *dst = C + (int64_t)row * ldc + col;
         if (vec_store) {
           *(v4i *)dst = v;
+        } else if (col + 3 < N) {
+          *(v4i_u *)dst = v;
         } else {
 #pragma unroll
           for (int r = 0; r < 4; r++)
@@ -1121,6 +1127,55 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Rows of K bytes at any address -> rows of Kp (a multiple of 16), zeros past K.
+// One thread per 16 bytes.  K >= 16.
+__global__ void __launch_bounds__(256)
+    pad_rows_i8(const int8_t *__restrict__ src, int64_t ld, int8_t *__restrict__ dst, int rows,
+                int K, int Kp) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int ch = Kp / 16;
+  if (i >= (int64_t)rows * ch) return;
+  const int64_t r = i / ch;
+  const int k = 16 * (int)(i - r * ch);
+  *(uint4 *)(dst + r * Kp + k) = k < K ? row16_any(src + r * ld, k, K) : make_uint4(0, 0, 0, 0);
+}
+
+// B[K,N] at any address -> B_T[N,Kp], zeros past K (Kp a multiple of 128, N >= 4).
+// A block takes 128 k x 128 n: a thread 16 k-rows of 4 columns (32 threads read
+// 128 bytes of a row side by side), transposed in registers; through LDS, eight
+// threads then write 128 bytes of a column side by side.
+__global__ void __launch_bounds__(256)
+    pad_transpose_i8(const int8_t *__restrict__ B, int64_t ldb, int8_t *__restrict__ BT, int K,
+                     int N, int Kp) {
+  __shared__ uint4 t[128][8];  // column n, 16-byte chunk of k (swizzled)
+  const int k0 = blockIdx.y * 128, n0 = blockIdx.x * 128;
+  {
+    const int nq = threadIdx.x & 31, kq = threadIdx.x >> 5;
+    const int gn = n0 + 4 * nq, back = max(0, min(gn + 4 - N, 3));
+    uint32_t d[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int gk = k0 + 16 * kq + r;
+      d[r] = gn < N && gk < K ? *(const u1any *)(B + (int64_t)gk * ldb + gn - back) >> (8 * back) : 0u;
+    }
+    uint32_t o[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      transpose4x4(d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3], o[0][q], o[1][q], o[2][q],
+                   o[3][q]);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      t[4 * nq + j][kq ^ (nq & 7)] = make_uint4(o[j][0], o[j][1], o[j][2], o[j][3]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int n = (threadIdx.x >> 3) + 32 * i, c = threadIdx.x & 7;
+    if (n0 + n < N)
+      *(uint4 *)(BT + (int64_t)(n0 + n) * Kp + k0 + 16 * c) = t[n][c ^ ((n >> 2) & 7)];
+  }
+}
+
 // C[z][r, c] = 0 for r < M, c < N (z: batch, sc elements apart).
 __global__ void __launch_bounds__(256)
     fill_i32_2d(int32_t *__restrict__ C, int64_t ldc, int M, int N, int64_t sc) {
@@ -1193,6 +1248,57 @@ int dispatch_tiles(const GemmArgs &g, hipStream_t st) {
 }
 
 template <bool BNK, bool AU8>
+int dispatch(const GemmArgs &g, hipStream_t st);
+
+// Products that the aligned kernels cannot read, large enough to pay for copies
+// of their operands with rows of a multiple of 128 bytes (B transposed on the
+// way): the kernels for B_T then run at their full rate.  Returns 1 where the
+// copies do not pay or their workspace cannot be had.
+//   B[K,N], from 2^29 products on: 717x2051x1533 18 us against 38 on the
+//   byte-aligned tiles (their loads are 4 bytes wide), 4095x4097x4099 110
+//   against 600, 1000^3 18 against 25.  B_T, from 2^32: 2000x5000x3001 70 us
+//   against 166, while 717x2051x1533 stays at 17 either way.
+template <bool BNK, bool AU8>
+int dispatch_padded(const GemmArgs &g, hipStream_t st) {
+  const int64_t work = (int64_t)g.M * g.N * g.K;
+  if (g.batch != 1 || g.scratch || g.M < 32 || g.K < 128 || g.N < 64 ||
+      work < (int64_t(1) << (BNK ? 32 : 29)))
+    return 1;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return 1;
+  const int Kp = (int)cdiv(g.K, 128) * 128;
+  const bool pad_a = g.K != Kp || g.lda % 16 != 0 || ((uintptr_t)g.A & 15) != 0;
+  const bool pad_b = !BNK || g.K != Kp || g.ldb % 16 != 0 || ((uintptr_t)g.B & 15) != 0;
+  const size_t ab = pad_a ? (size_t)g.M * Kp : 0, bb = pad_b ? (size_t)g.N * Kp : 0;
+  void *ws = nullptr;
+  if (workspace(st, ab + bb, &ws, 5) != SIMP_RT_OK) {
+    clear_error();
+    return 1;
+  }
+  int8_t *a8 = (int8_t *)ws, *b8 = a8 + ab;
+  GemmArgs h = g;
+  h.K = Kp;
+  if (pad_a) {
+    hipLaunchKernelGGL(pad_rows_i8, dim3((unsigned)cdiv((int64_t)g.M * (Kp / 16), 256)), dim3(256), 0,
+                       st, g.A, g.lda, a8, g.M, g.K, Kp);
+    h.A = a8;
+    h.lda = Kp;
+  }
+  if (pad_b) {
+    if (BNK)
+      hipLaunchKernelGGL(pad_rows_i8, dim3((unsigned)cdiv((int64_t)g.N * (Kp / 16), 256)), dim3(256),
+                         0, st, g.B, g.ldb, b8, g.N, g.K, Kp);
+    else
+      hipLaunchKernelGGL(pad_transpose_i8, dim3((unsigned)cdiv(g.N, 128), (unsigned)(Kp / 128)),
+                         dim3(256), 0, st, g.B, g.ldb, b8, g.K, g.N, Kp);
+    h.B = b8;
+    h.ldb = Kp;
+  }
+  SIMP_HIP(hipGetLastError());
+  return dispatch<true, AU8>(h, st);
+}
+
+template <bool BNK, bool AU8>
 int dispatch(const GemmArgs &g, hipStream_t st) {
   if (g.M == 0 || g.N == 0 || g.batch == 0) return SIMP_RT_OK;
   const int64_t cus = num_cus();
@@ -1223,6 +1329,10 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
   const bool b_ok = BNK ? (g.ldb % 16 == 0 && ((uintptr_t)g.B & 15) == 0 && g.sb % 16 == 0)
                         : (g.N % 4 == 0 && g.ldb % 4 == 0 && ((uintptr_t)g.B & 3) == 0 &&
                            g.sb % 4 == 0);
+  if (!a_ok || !b_ok) {
+    const int rc = dispatch_padded<BNK, AU8>(g, st);
+    if (rc != 1) return rc;
+  }
   if ((!a_ok || !b_ok) && g.K >= 16 && (BNK || g.N >= 4))
     return dispatch_tiles<BNK, AU8, true>(g, st);
   if (!a_ok || !b_ok) {
@@ -1233,9 +1343,12 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     SIMP_HIP(hipGetLastError());
     return SIMP_RT_OK;
   }
-  if (g.batch == 1 && tiles(256, 256) >= cus && g.N % 16 == 0) {
+  // (the kernels for B_T read whole rows and take any N: column by column
+  // stores where a row of C does not end with a 16-byte one)
+  const bool any_n = BNK && g.K % 128 == 0;
+  if (g.batch == 1 && tiles(256, 256) >= cus && (any_n || g.N % 16 == 0)) {
     const int tm = (int)cdiv(g.M, 256), tn = (int)cdiv(g.N, 256);
-    const int vec = g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
+    const int vec = g.N % 4 == 0 && g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
     // persistent grid: one workgroup per CU, a multiple of 8 (XCD round-robin)
     const int grid = (int)std::max<int64_t>(8, std::min<int64_t>(cus, (int64_t)tm * tn) / 8 * 8);
     // B[K,N] with 16-byte aligned rows is read in place by gemm_i8_dma
@@ -1339,9 +1452,9 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     // A deeper prefetch spreads an XCD's CUs over more operand lines than its
     // L2 keeps; a shallower one exposes the load latency when a CU has the
     // memory system to itself for longer (long K, part of the chip idle).
-    const bool ok = g.batch == 1 && g.K % 128 == 0 && g.N % 16 == 0 && g.ldb % 16 == 0 &&
+    const bool ok = g.batch == 1 && g.K % 128 == 0 && (any_n || g.N % 16 == 0) && g.ldb % 16 == 0 &&
                     ((uintptr_t)g.B & 15) == 0;
-    const int vec = g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
+    const int vec = g.N % 4 == 0 && g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
     auto ring = [&](auto bm, auto slots) {
       constexpr int BM = decltype(bm)::value, SL = decltype(slots)::value;
       const int tm = (int)cdiv(g.M, BM), tn = (int)cdiv(g.N, BM);

@@ -8,9 +8,11 @@ import simplang_amd as sa
 pytestmark = pytest.mark.gpu
 
 # K around 16, 32 and the 128-deep step, with remainders; N % 4 of 0 to 3, below
-# and above a tile; one and several K splits; 128x128 tiles (2049x2055)
+# and above a tile; one and several K splits; 128x128 tiles (2049x2055); operands copied to padded rows
+# (the last three: 64x64, 128x128 and 256x256 tiles)
 SHAPES = [(1, 5, 17), (2, 3, 40), (3, 4, 16), (5, 6, 15), (33, 67, 31), (40, 64, 129), (64, 131, 255),
-          (100, 258, 1533), (7, 4099, 1025), (2049, 2055, 100), (129, 130, 143)]
+          (100, 258, 1533), (7, 4099, 1025), (2049, 2055, 100), (129, 130, 143),
+          (717, 803, 1001), (1300, 1283, 2601), (4100, 4097, 260)]
 
 
 @pytest.mark.parametrize("u8", [False, True])
@@ -26,7 +28,7 @@ def test_any_size_and_alignment(dev, M, N, K, nt, u8):
           (True, False): sa.tensor_matmul_nt_i8, (True, True): sa.matmul_nt_u8s8_i32}[nt, u8]
     want = (a.astype(np.float64) @ (b.T if nt else b).astype(np.float64)).astype(np.int64)
     # dense (the last rows end with the allocation), and views with odd pitches
-    for off, pad in ((0, 0), (1, 2), (3, 13)):
+    for off, pad in ((0, 0), (1, 2), (3, 13)) if M < 4000 else ((1, 2),):
         at = torch.zeros(M, K + off + pad, dtype=torch.uint8 if u8 else torch.int8)
         bt = torch.full((b.shape[0], b.shape[1] + off + pad), 77, dtype=torch.int8)
         at[:, off:off + K] = torch.from_numpy(a)
