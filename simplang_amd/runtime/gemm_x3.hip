@@ -138,7 +138,7 @@ struct X3Args {
 //     1.1 to 1.4); mid sizes the splitting next to it (128x2048x8192 31.5 us
 //     against 43.0, 301x1537x2003 with B_T 22.8 against 315 for the SIMT kernel
 //     that odd sizes took; a copy without the operand loads runs as long).  W4:
-//     the nibble conversion and the scaling (200x3200x8640: 78 us; one thread
+//     the nibble conversion and the scaling (200x3200x8640: 61 us; one thread
 //     per output took 131 ms).
 //   * A part that overflows or an infinite or NaN operand makes its products
 //     NaN where fp32 arithmetic may give an infinity: tiles with a non-finite
@@ -291,28 +291,36 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
   // the sign of A in step s and of the carried sums
   auto sign = [&](int s) { return CARRY && ((s - s0) >> 2) & 1 ? -1.f : 1.f; };
   auto compute = [&](int buf, const Frag &f, float sg) {
+    // two row blocks at a time: the MFMAs of one sum are 2 NT apart
+    constexpr int R = MT % 2 == 0 ? 2 : 1;
     if constexpr (W4) {
 #pragma unroll
-      for (int i = 0; i < MT; i++) {
-        const Planes p = frag(buf, i);
-        v4f d[NT];
+      for (int i = 0; i < MT; i += R) {
+        Planes p[R];
+        v4f d[R][NT];
 #pragma unroll
-        for (int j = 0; j < NT; j++) d[j] = mfma_bf16(p.l, f.w[j], v4f{0.f, 0.f, 0.f, 0.f});
+        for (int q = 0; q < R; q++) p[q] = frag(buf, i + q);
+        auto mul = [&](b8 Planes::*y, auto zero) {
 #pragma unroll
-        for (int j = 0; j < NT; j++) d[j] = mfma_bf16(p.m, f.w[j], d[j]);
+          for (int q = 0; q < R; q++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) d[j] = mfma_bf16(p.h, f.w[j], d[j]);
+            for (int j = 0; j < NT; j++)
+              d[q][j] = mfma_bf16(p[q].*y, f.w[j],
+                                  decltype(zero)::value ? v4f{0.f, 0.f, 0.f, 0.f} : d[q][j]);
+        };
+        mul(&Planes::l, std::true_type{});
+        mul(&Planes::m, std::false_type{});
+        mul(&Planes::h, std::false_type{});
 #pragma unroll
-        for (int j = 0; j < NT; j++) {
+        for (int q = 0; q < R; q++)
 #pragma unroll
-          for (int e = 0; e < 4; e++)
-            acc[i][j][e] = fmaf(sg < 0.f ? -f.s[j] : f.s[j], d[j][e], acc[i][j][e]);
-        }
+          for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              acc[i + q][j][e] = fmaf(sg < 0.f ? -f.s[j] : f.s[j], d[q][j][e], acc[i + q][j][e]);
       }
     } else {
-      // two row blocks at a time and small parts first: the MFMAs of one sum
-      // are 2 NT apart
-      constexpr int R = MT % 2 == 0 ? 2 : 1;
+      // small parts first
 #pragma unroll
       for (int i = 0; i < MT; i += R) {
         Planes p[R];
@@ -533,7 +541,7 @@ __global__ void __launch_bounds__(256)
 // CUs costs its steps and about four more to fill and drain its pipeline; the
 // partial sums cost a launch (about three steps' time) and their traffic (a
 // step is about 1 us, in which 4 MB go by).  Measured (W4, 200 x 3200 -> 8640,
-// 136 tiles: 1 / 3 / 4 / 6 splits 120 / 77 / 90 / 87 us; fp32 128 x 2048 x 8192,
+// 68 tiles: 3 / 6 / 7 splits 61 / 72 / 71 us; fp32 128 x 2048 x 8192,
 // 128 tiles: 1 / 2 / 4 splits 70 / 39 / 39 us).
 int pick_splits(int64_t tiles, int steps, int64_t mn, int64_t cus) {
   int best = 1;
@@ -639,10 +647,15 @@ int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, 
   (fmt == X3Fmt::kN ? go_x3<MT, NT, NW, kBKN, __VA_ARGS__>(a, split, must, st)          \
                     : go_x3<MT, NT, NW, kBNK, __VA_ARGS__>(a, split, must, st))
   if (fmt == X3Fmt::kW4) {
-    if (M <= 16) return go_x3<1, 2, 4, kBW4, 4>(a, split, must, st);
-    if (M <= 32) return go_x3<2, 2, 4, kBW4, 4>(a, split, must, st);
-    if (M <= 64) return go_x3<4, 2, 4, kBW4, 4>(a, split, must, st);
-    return go_x3<8, 2, 4, kBW4, 4>(a, split, must, st);
+    // 256 columns on 8 waves, which split A half as often, from 24 tiles on (200x
+    // 3200x8640 61 us against 77, 64x3200x32000 60 against 65); fewer leave too
+    // few workgroups to a split of K (64x8640x3200 28.8 against 26.8, 64x2048x2048
+    // 19 against 15)
+#define X3_W4(MT)                                                          \
+  (cdiv(M, 16 * MT) * cdiv(N, 256) >= 24 ? go_x3<MT, 2, 8, kBW4, 4>(a, split, must, st) \
+                                         : go_x3<MT, 2, 4, kBW4, 4>(a, split, must, st))
+    return M <= 16 ? X3_W4(1) : M <= 32 ? X3_W4(2) : M <= 64 ? X3_W4(4) : X3_W4(8);
+#undef X3_W4
   }
   // 16- and 32-row tiles for few rows (24x2048x8192: 16 us on 32x128 tiles of 8
   // waves, 22 on 32x64 of 4, 20 on 64x128)
