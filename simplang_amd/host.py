@@ -130,7 +130,7 @@ def _check_float(fn: str, errors_before: int, r: float) -> float:
 # ------------------------------------------------------------------ operands
 
 def _is_torch(x) -> bool:
-    return type(x).__module__.startswith("torch")
+    return type(x).__module__[:5] == "torch"
 
 
 def _ptr_stride(x):
@@ -161,6 +161,11 @@ def _ptr_stride(x):
 
 
 def desc2(x):
+    if _is_torch(x):  # the usual operand, without the general path's second look at it
+        shape, st = x.shape, x.stride()
+        if len(shape) == 2 and st[1] == 1:
+            p = x.data_ptr()
+            return [p, p, 0, shape[0], shape[1], st[0], 1]
     p, st0, shape = _ptr_stride(x)
     if len(shape) != 2:
         raise ValueError("expected a rank-2 tensor")
@@ -186,6 +191,11 @@ def descn(x, rank: int):
 
 
 def desc1(x):
+    if _is_torch(x):
+        shape = x.shape
+        if len(shape) == 1 and x.stride(0) == 1:
+            p = x.data_ptr()
+            return [p, p, 0, shape[0], 1]
     p, _, shape = _ptr_stride(x)
     n = 1
     for s in shape:
