@@ -426,7 +426,9 @@ int32_t simp_rt_llama_forward(simp_rt_llama *model, int64_t token, int64_t pos, 
 /* Greedy generation (strict-'>' argmax, generate_stories110M.cpp:73-83): runs
  * the prompt then n_new sampled tokens; out_tokens[n_prompt + n_new] (host)
  * receives prompt and samples.  use_graph != 0 replays one captured HIP graph
- * per step with the token/position state kept on the device. */
+ * per step with the token/position state kept on the device.  From nine prompt
+ * tokens on, all but the last are taken through the layers together (the same
+ * K/V rows up to rounding) instead of one step each. */
 int32_t simp_rt_llama_generate(simp_rt_llama *model, const int32_t *prompt, int64_t n_prompt,
                                int64_t n_new, int32_t *out_tokens, int32_t use_graph);
 

@@ -1211,7 +1211,8 @@ int capture_step(LlamaModel &m, int mode) {
 // Runs the first n tokens of the prompt (already on the device) as rows of
 // matrices; *done receives how many of them it took, n or 0 (shapes that the
 // row kernels do not take, no memory for the activations, or too few tokens:
-// a pass costs about as much as six steps, 110M 1.9 ms, 3B W4 5 ms).
+// a pass costs about as much as five steps: 110M 1.4 ms for 199 tokens, 3B W4
+// 4.4 ms for 31, against 0.31 and 0.88 ms a step).
 constexpr int64_t kPrefillMin = 8, kPrefillRows = 512;
 int prefill_prompt(LlamaModel &m, int64_t n, int64_t *done) {
   *done = 0;

@@ -1265,7 +1265,11 @@ int dispatch_padded(const GemmArgs &g, hipStream_t st) {
       work < (int64_t(1) << (BNK ? 32 : 29)))
     return 1;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return 1;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+    (void)hipGetLastError();  // the launch check must not see it
+    return 1;
+  }
+  if (cs != hipStreamCaptureStatusNone) return 1;  // a graph must not hold the workspace
   const int Kp = (int)cdiv(g.K, 128) * 128;
   const bool pad_a = g.K != Kp || g.lda % 16 != 0 || ((uintptr_t)g.A & 15) != 0;
   const bool pad_b = !BNK || g.K != Kp || g.ldb % 16 != 0 || ((uintptr_t)g.B & 15) != 0;
@@ -1273,6 +1277,7 @@ int dispatch_padded(const GemmArgs &g, hipStream_t st) {
   void *ws = nullptr;
   if (workspace(st, ab + bb, &ws, 5) != SIMP_RT_OK) {
     clear_error();
+    (void)hipGetLastError();
     return 1;
   }
   int8_t *a8 = (int8_t *)ws, *b8 = a8 + ab;

@@ -574,6 +574,7 @@ int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
   if (splits > 1) {
     if (may_split && workspace(st, sizeof(float) * (size_t)splits * a.M * a.N, (void **)&a.P, 3) != SIMP_RT_OK) {
       clear_error();
+      (void)hipGetLastError();  // of the allocation: the launch check must not see it
       may_split = false;
     }
     if (!may_split) {
@@ -609,7 +610,9 @@ int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
 // may replace.
 bool capturing(hipStream_t st) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // the launch check must not see it
+  return true;
 }
 
 }  // namespace
