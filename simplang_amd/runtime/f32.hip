@@ -9,7 +9,9 @@
 // n == 1 (every LLaMA decode projection, stories110M.sl:77-83) is an HBM-bound
 // GEMV: one wave per output row at a time, lanes along K with 16-byte loads, x
 // held in registers for the whole kernel, the next row's loads in flight while
-// the current row is reduced.  n > 1 runs an LDS-tiled fp32 GEMM.
+// the current row is reduced.  Single products of more than 16 rows, or with
+// operands that 16-byte loads cannot read, run on the split-bf16 kernel
+// (gemm_x3.hip); batches and few rows on the fp32 MFMA kernels here.
 #include <algorithm>
 #include <type_traits>
 

@@ -135,10 +135,10 @@ struct X3Args {
 //   * What bounds it: large products the MFMA rate the chip sustains (4096^3: 686
 //     us against 1020 for the fp32 MFMA kernel; the MFMA pipe is busy 65% of the
 //     cycles at 1.75 GHz, 1.2 PFLOP/s of bf16, where a bf16 library GEMM reaches
-//     1.1 to 1.4); mid sizes the splitting next to it (128x2048x8192 31.5 us
-//     against 43.0, 301x1537x2003 with B_T 22.8 against 315 for the SIMT kernel
+//     1.1 to 1.4); mid sizes the splitting next to it (128x2048x8192 32.8 us
+//     against 43.0, 301x1537x2003 with B_T 23.4 against 314 for the SIMT kernel
 //     that odd sizes took; a copy without the operand loads runs as long).  W4:
-//     the nibble conversion and the scaling (200x3200x8640: 61 us; one thread
+//     the nibble conversion and the scaling (200x3200x8640: 58 us; one thread
 //     per output took 131 ms).
 //   * A part that overflows or an infinite or NaN operand makes its products
 //     NaN where fp32 arithmetic may give an infinity: tiles with a non-finite
