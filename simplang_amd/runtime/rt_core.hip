@@ -17,6 +17,7 @@
 
 #include <atomic>
 #include "rt_internal.h"
+#include "workspace.h"
 
 namespace simp {
 
@@ -77,50 +78,48 @@ int num_cus() {
 }
 
 namespace {
-struct WsKey {
-  int dev;
-  hipStream_t stream;
-  int slot;
-  bool operator<(const WsKey &o) const {
-    if (dev != o.dev) return dev < o.dev;
-    if (stream != o.stream) return (uintptr_t)stream < (uintptr_t)o.stream;
-    return slot < o.slot;
+struct HipMem {
+  using Stream = hipStream_t;
+  bool capturing(hipStream_t st) const {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // the launch check must not see it
+    return false;
+  }
+  void *alloc(size_t bytes) const {
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  bool sync(hipStream_t st) const { return check(hipStreamSynchronize(st), "hipStreamSynchronize"); }
+  bool free(void *p) const { return check(hipFree(p), "hipFree"); }
+
+ private:
+  static bool check(hipError_t e, const char *what) {
+    if (e != hipSuccess) hip_fail(e, what);
+    return e == hipSuccess;
   }
 };
-struct WsBuf {
-  void *ptr = nullptr;
-  size_t bytes = 0;
-};
-std::map<WsKey, WsBuf> g_ws;
+WsPool<HipMem> &ws_pool() {
+  static auto *pool = new WsPool<HipMem>();  // outlives the threads that may call at exit
+  return *pool;
+}
 }  // namespace
 
 int workspace(hipStream_t stream, size_t bytes, void **ptr, int slot) {
   int dev = ensure_device();
   if (dev < 0) return dev;
-  std::lock_guard<std::mutex> lk(g_mu);
-  WsBuf &b = g_ws[WsKey{dev, stream, slot}];
-  if (b.bytes < bytes) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+  switch (ws_pool().get({dev, stream, slot}, bytes, ptr)) {
+    case WsStatus::kOk: return SIMP_RT_OK;
+    case WsStatus::kCapturing:
       return set_error(SIMP_RT_EUNSUPPORTED,
                        "workspace of %zu bytes needed while the stream is being captured; "
                        "make one uncaptured call of the same size on this stream first", bytes);
-    if (b.ptr) {
-      SIMP_HIP(hipStreamSynchronize(stream));  // earlier calls may still read it
-      SIMP_HIP(hipFree(b.ptr));
-      b.ptr = nullptr;
-      b.bytes = 0;
-    }
-    size_t want = std::max(bytes, (size_t)1 << 20);
-    hipError_t e = hipMalloc(&b.ptr, want);
-    if (e != hipSuccess) {
-      b.ptr = nullptr;
-      return set_error(SIMP_RT_ENOMEM, "workspace of %zu bytes: %s", want, hipGetErrorString(e));
-    }
-    b.bytes = want;
+    case WsStatus::kNoMemory:
+      return set_error(SIMP_RT_ENOMEM, "workspace of %zu bytes: out of device memory", bytes);
+    default: return SIMP_RT_EHIP;
   }
-  *ptr = b.ptr;
-  return SIMP_RT_OK;
 }
 
 // Looks p up in the registry; returns the device address or nullptr.

@@ -135,10 +135,11 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 int num_cus();
 
 // Library-owned device scratch for (current device, stream, slot), grown on
-// demand and kept until the process ends.  Calls on one stream are ordered, so
-// they may share it; calls on different streams get different buffers.  Slot 0
-// belongs to the int8 GEMM dispatch; an entry point that stages operands for it
-// (the i4 product) uses slot 1.
+// demand and kept until the process ends (workspace.h).  Calls on one stream are
+// ordered, so they may share it; calls on different streams get different
+// buffers, and captured calls others than uncaptured ones, which no later call
+// frees.  Slot 0 belongs to the int8 GEMM dispatch; an entry point that stages
+// operands for it (the i4 product) uses slot 1.
 int workspace(hipStream_t stream, size_t bytes, void **ptr, int slot = 0);
 
 // Optional per-kernel timing (simp_rt_timing): while enabled, a KernelTimer
