@@ -57,7 +57,8 @@ int bench_program(int N, int32_t *checksum) {
   const size_t nn = (size_t)N * N;
   // A [N,N] i8 | B [N,N] i8 | C [N,N] i32 | checksum; slot 2 is this file's
   void *ws = nullptr;
-  int rc = workspace(st, 6 * nn + 256, &ws, 2);
+  Workspace lease;
+  int rc = lease.get(st, 6 * nn + 256, &ws, 2);
   if (rc) return rc;
   int8_t *A = (int8_t *)ws, *B = A + nn;
   int32_t *C = (int32_t *)(B + nn);

@@ -526,8 +526,9 @@ int launch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, int
   const int k_span = (int)(cdiv(nkt, splits) * 16);
   splits = cdiv(K, k_span);
   float *P = nullptr;
+  Workspace ws;
   if (splits > 1) {
-    int rc = workspace(st, sizeof(float) * (size_t)batch * splits * M * N, (void **)&P, 3);
+    int rc = ws.get(st, sizeof(float) * (size_t)batch * splits * M * N, (void **)&P, 3);
     if (rc) return rc;
   }
   KernelTimer kt(st, "gemm_f32_mfma");

@@ -1275,7 +1275,8 @@ int dispatch_padded(const GemmArgs &g, hipStream_t st) {
   const bool pad_b = !BNK || g.K != Kp || g.ldb % 16 != 0 || ((uintptr_t)g.B & 15) != 0;
   const size_t ab = pad_a ? (size_t)g.M * Kp : 0, bb = pad_b ? (size_t)g.N * Kp : 0;
   void *ws = nullptr;
-  if (workspace(st, ab + bb, &ws, 5) != SIMP_RT_OK) {
+  Workspace lease;
+  if (lease.get(st, ab + bb, &ws, 5) != SIMP_RT_OK) {
     clear_error();
     (void)hipGetLastError();
     return 1;
@@ -1376,6 +1377,7 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     GemmArgs h = g;
     const size_t cs_bytes = AU8 && !csk ? ((size_t)g.N * 4 + 255) / 256 * 256 : 0;
     void *ws = nullptr;
+    Workspace lease;
     const size_t need = cs_bytes + (BNK || direct ? 0 : (size_t)g.K * g.N);
     if (g.scratch) {
       if (need > g.scratch_bytes)
@@ -1385,7 +1387,7 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
                          g.scratch_bytes);
       ws = g.scratch;
     } else if (need) {
-      int rc = workspace(st, need, &ws);
+      int rc = lease.get(st, need, &ws);
       if (rc) return rc;
     }
     int32_t *colsum = AU8 && !csk ? (int32_t *)ws : nullptr;
@@ -1849,7 +1851,8 @@ int32_t simp_rt_tensor_matmul_i4(
   auto al = [](size_t x) { return (x + 255) / 256 * 256; };
   const size_t a8 = al((size_t)M * Kp), b8 = al((size_t)N * Kp), c32 = al((size_t)M * N * 4);
   void *ws = nullptr;
-  if ((rc = workspace(st, a8 + b8 + c32, &ws, 1))) return rc;
+  Workspace lease;
+  if ((rc = lease.get(st, a8 + b8 + c32, &ws, 1))) return rc;
   int8_t *A8 = (int8_t *)ws, *BT8 = A8 + a8;
   int32_t *C32 = (int32_t *)(BT8 + b8);
   hipLaunchKernelGGL(unpack_i4_rows, dim3((unsigned)cdiv(M * (Kp / 16), 256)), dim3(256), 0, st,

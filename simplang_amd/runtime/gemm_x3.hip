@@ -571,8 +571,9 @@ int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
   const int steps = (int)cdiv(a.K, 32);
   int splits = pick_splits(tm * tn, steps, (int64_t)a.M * a.N, cus);
   a.P = nullptr;
+  Workspace ws;
   if (splits > 1) {
-    if (may_split && workspace(st, sizeof(float) * (size_t)splits * a.M * a.N, (void **)&a.P, 3) != SIMP_RT_OK) {
+    if (may_split && ws.get(st, sizeof(float) * (size_t)splits * a.M * a.N, (void **)&a.P, 3) != SIMP_RT_OK) {
       clear_error();
       (void)hipGetLastError();  // of the allocation: the launch check must not see it
       may_split = false;

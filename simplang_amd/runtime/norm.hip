@@ -307,7 +307,8 @@ int launch_rmsnorm(const float *x, const float *w, float *out, int n, float eps,
   if (n >= kBigNorm) {
     const unsigned g = big_grid(n);
     float *part = nullptr;
-    int rc = workspace(st, sizeof(float2) * g, (void **)&part, 4);
+    Workspace ws;
+    int rc = ws.get(st, sizeof(float2) * g, (void **)&part, 4);
     if (rc) return rc;
     const bool vec = (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
     hipLaunchKernelGGL(sumsq_parts_k, dim3(g), dim3(256), 0, st, x, (int64_t)n, part, vec);
@@ -373,7 +374,8 @@ int32_t simp_rt_softmax(const float *in_alloc, const float *in, int64_t in_doff,
   if (size >= kBigNorm) {
     const unsigned g = big_grid(size);
     float2 *part = nullptr;
-    if ((rc = workspace(st, sizeof(float2) * g, (void **)&part, 4))) return rc;
+    Workspace ws;
+    if ((rc = ws.get(st, sizeof(float2) * g, (void **)&part, 4))) return rc;
     const bool vec = (((uintptr_t)oi.dev() | (uintptr_t)oo.dev()) & 15) == 0;
     hipLaunchKernelGGL(softmax_parts_k, dim3(g), dim3(256), 0, st, (const float *)oi.dev(),
                        (int64_t)size, part, vec);

@@ -107,10 +107,13 @@ WsPool<HipMem> &ws_pool() {
 }
 }  // namespace
 
-int workspace(hipStream_t stream, size_t bytes, void **ptr, int slot) {
+int Workspace::get(hipStream_t stream, size_t bytes, void **ptr, int slot) {
+  static thread_local char here;  // its address names the thread
   int dev = ensure_device();
   if (dev < 0) return dev;
-  switch (ws_pool().get({dev, stream, slot}, bytes, ptr)) {
+  release();
+  const void *thread = stream == hipStreamPerThread ? &here : nullptr;
+  switch (ws_pool().get({dev, stream, thread, slot}, bytes, ptr, lease_)) {
     case WsStatus::kOk: return SIMP_RT_OK;
     case WsStatus::kCapturing:
       return set_error(SIMP_RT_EUNSUPPORTED,

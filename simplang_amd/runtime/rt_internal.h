@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -138,9 +139,20 @@ int num_cus();
 // demand and kept until the process ends (workspace.h).  Calls on one stream are
 // ordered, so they may share it; calls on different streams get different
 // buffers, and captured calls others than uncaptured ones, which no later call
-// frees.  Slot 0 belongs to the int8 GEMM dispatch; an entry point that stages
-// operands for it (the i4 product) uses slot 1.
-int workspace(hipStream_t stream, size_t bytes, void **ptr, int slot = 0);
+// frees.  The object keeps other threads' calls away from the buffer, so it
+// lives until the call's last launch that uses it.  Slot 0 belongs to the int8
+// GEMM dispatch; an entry point that stages operands for it (the i4 product) uses
+// slot 1.
+class Workspace {
+ public:
+  int get(hipStream_t stream, size_t bytes, void **ptr, int slot = 0);
+  void release() {
+    if (lease_.owns_lock()) lease_.unlock();
+  }
+
+ private:
+  std::unique_lock<std::mutex> lease_;
+};
 
 // Optional per-kernel timing (simp_rt_timing): while enabled, a KernelTimer
 // brackets the launches between its construction and stop() with HIP events on

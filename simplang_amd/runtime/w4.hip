@@ -648,8 +648,9 @@ int launch_w4s(const uint8_t *W, int64_t ldw, const float *S, int64_t lds, const
     const int chunks = (int)cdiv(nck, std::min(want, nck));
     const int parts = (int)cdiv(nck, chunks);
     float *P = nullptr;
+    Workspace ws;
     if (parts > 1) {
-      int rc = workspace(st, sizeof(float) * (size_t)parts * M * N, (void **)&P, 2);
+      int rc = ws.get(st, sizeof(float) * (size_t)parts * M * N, (void **)&P, 2);
       if (rc) return rc;
     }
     KernelTimer kt(st, "w4s_h16");

@@ -14,6 +14,12 @@
 //     old one stays behind for its graphs.  The eager buffer that such a call
 //     needs is made twice as large as the graphs' one, so what stays behind
 //     adds up to less than the buffer in use.
+//
+// A call that writes scratch with one launch and reads it with a later one holds
+// a Lease from the lookup to its last launch: no other thread's call on the same
+// stream then puts its launches in between, or frees the buffer by growing it.
+// Leases nest in the order of the slots' users (a product that stages operands
+// in one slot runs another product on them), never in a circle.
 #pragma once
 
 #include <algorithm>
@@ -36,14 +42,18 @@ template <class Mem>
 class WsPool {
  public:
   using Stream = typename Mem::Stream;
-  using Key = std::tuple<int, Stream, int>;  // device, stream, slot
+  // device, stream, the thread where the stream's handle names one per thread
+  // (else null), slot
+  using Key = std::tuple<int, Stream, const void *, int>;
+  using Lease = std::unique_lock<std::mutex>;
 
   explicit WsPool(Mem mem = Mem()) : mem_(mem) {}
 
-  // A buffer of at least `bytes` for the next launches on the key's stream.
-  WsStatus get(const Key &key, size_t bytes, void **ptr) {
-    std::lock_guard<std::mutex> lk(mu_);
-    Entry &e = entries_[key];
+  // A buffer of at least `bytes` for the launches on the key's stream that the
+  // caller makes while it holds `lease`.
+  WsStatus get(const Key &key, size_t bytes, void **ptr, Lease &lease) {
+    Entry &e = entry(key);
+    lease = Lease(e.mu);
     const Stream st = std::get<1>(key);
     if (mem_.capturing(st)) {
       if (e.graph.bytes < bytes) {
@@ -79,8 +89,13 @@ class WsPool {
     size_t bytes = 0;
   };
   struct Entry {
+    std::mutex mu;
     Buf eager, graph;
   };
+  Entry &entry(const Key &key) {  // entries stay where they are
+    std::lock_guard<std::mutex> lk(mu_);
+    return entries_[key];
+  }
   Mem mem_;
   std::mutex mu_;
   std::map<Key, Entry> entries_;

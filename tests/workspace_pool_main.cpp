@@ -2,7 +2,8 @@
 // that counts: run by test_workspace_pool.py.
 #include <cstdio>
 #include <cstdlib>
-#include <set>
+#include <thread>
+#include <vector>
 
 #include "workspace.h"
 
@@ -18,7 +19,14 @@ using namespace simp;
 
 constexpr size_t MB = size_t(1) << 20;
 
+struct Event {  // of a stream: kernels, and frees (which follow a drain)
+  char what;
+  void *buf;
+  int who;
+};
 struct State {
+  std::mutex mu;
+  std::vector<Event> stream;
   bool capturing = false;
   size_t limit = ~size_t(0), held = 0, syncs = 0, allocs = 0;
   std::map<void *, size_t> live;
@@ -28,14 +36,20 @@ struct FakeMem {
   State *s;
   bool capturing(int) const { return s->capturing; }
   void *alloc(size_t n) const {
+    std::lock_guard<std::mutex> lk(s->mu);
     if (s->held + n > s->limit) return nullptr;
     void *p = (void *)(4096 * ++s->allocs);  // an address of its own, never read
     s->live[p] = n;
     s->held += n;
     return p;
   }
-  bool sync(int) const { return ++s->syncs, true; }
+  bool sync(int) const {
+    std::lock_guard<std::mutex> lk(s->mu);
+    return ++s->syncs, true;
+  }
   bool free(void *p) const {
+    std::lock_guard<std::mutex> lk(s->mu);
+    s->stream.push_back({'f', p, -1});
     CHECK(s->live.count(p));
     s->held -= s->live[p];
     s->live.erase(p);
@@ -48,7 +62,8 @@ void *get(Pool &p, State &s, bool capturing, size_t bytes, WsStatus want = WsSta
           int slot = 3) {
   s.capturing = capturing;
   void *ptr = nullptr;
-  CHECK(p.get(Pool::Key{0, stream, slot}, bytes, &ptr) == want);
+  Pool::Lease lease;
+  CHECK(p.get(Pool::Key{0, stream, nullptr, slot}, bytes, &ptr, lease) == want);
   CHECK(want != WsStatus::kOk || s.live.at(ptr) >= bytes);
   return ptr;
 }
@@ -108,10 +123,44 @@ void no_memory() {
   CHECK(s.held == 5 * MB);
 }
 
+// Threads on one stream: each call's launches stay together, and no buffer is
+// freed between a lookup and the launches that use it.
+void threads_share_a_stream() {
+  State s;
+  Pool p(FakeMem{&s});
+  auto enqueue = [&](char what, void *buf, int who) {
+    std::lock_guard<std::mutex> lk(s.mu);
+    s.stream.push_back({what, buf, who});
+  };
+  std::vector<std::thread> ts;
+  for (int t = 0; t < 4; t++)
+    ts.emplace_back([&, t] {
+      for (int i = 0; i < 500; i++) {
+        void *buf = nullptr;
+        Pool::Lease lease;
+        CHECK(p.get(Pool::Key{0, 0, nullptr, 5}, (size_t)(1 + (7 * i + t) % 500) * (MB / 8), &buf,
+                    lease) == WsStatus::kOk);
+        enqueue('w', buf, t);
+        std::this_thread::yield();
+        enqueue('r', buf, t);
+      }
+    });
+  for (auto &t : ts) t.join();
+  std::map<void *, int> holds;  // buffer -> whose data, -1 once freed
+  for (const Event &e : s.stream) {
+    if (e.what == 'f') holds[e.buf] = -1;
+    CHECK(e.what != 'w' || !holds.count(e.buf) || holds[e.buf] != -1);
+    if (e.what == 'w') holds[e.buf] = e.who;
+    CHECK(e.what != 'r' || holds[e.buf] == e.who);
+  }
+  CHECK(s.stream.size() > 4000 && s.syncs > 0);
+}
+
 int main() {
   graphs_keep_their_buffers();
   capture_needs_a_warm_up();
   what_stays_behind_is_bounded();
   no_memory();
+  threads_share_a_stream();
   std::puts("ok");
 }
