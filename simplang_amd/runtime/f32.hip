@@ -503,10 +503,11 @@ __global__ void __launch_bounds__(256)
   *o = beta != 0.f ? *o + v : v;
 }
 
+// or_one: 1 instead of an error when there is no workspace for the K splits.
 template <int BM, int BN, int WGM, int WGN, bool BT, int BK = 16>
 int launch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, int64_t ldb,
                     int64_t sb, float *C, int64_t ldc, int64_t sc, int M, int N, int K, int batch,
-                    float beta, hipStream_t st) {
+                    float beta, hipStream_t st, bool or_one = false) {
   const int64_t tiles_n = cdiv(N, BN), tiles = cdiv(M, BM) * tiles_n;
   if (tiles > INT32_MAX)
     return set_error(SIMP_RT_EUNSUPPORTED, "gemm: %lld output tiles exceed one launch",
@@ -528,8 +529,12 @@ int launch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, int
   float *P = nullptr;
   Workspace ws;
   if (splits > 1) {
-    int rc = ws.get(st, sizeof(float) * (size_t)batch * splits * M * N, (void **)&P, 3);
-    if (rc) return rc;
+    const size_t bytes = sizeof(float) * (size_t)batch * splits * M * N;
+    if (or_one) {
+      if (!ws.try_get(st, bytes, (void **)&P, 3)) return 1;
+    } else if (int rc = ws.get(st, bytes, (void **)&P, 3)) {
+      return rc;
+    }
   }
   KernelTimer kt(st, "gemm_f32_mfma");
   hipLaunchKernelGGL((gemm_f32_mfma<BM, BN, WGM, WGN, BT, BK>),
@@ -593,18 +598,26 @@ int dispatch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, i
   // 24x768x768 9.2 us against 9.8, 128x768x768 with B_T 10.5 against 11.4
   const int64_t kn = (int64_t)K * N;
   const bool small = M <= 32 ? kn < (1 << 20) : BT && M <= 128 && kn <= (5 << 18);
-  if (batch == 1 && M > 16 && !one_round && !small) {
+  const bool x3 = batch == 1 && M > 16 && !one_round && !small;
+  auto split_product = [&](bool must) {
     const X3Mat b{B, nullptr, N};
     // carried sums where the ring kernel would carry its own through all of K;
     // the smaller shapes, whose K it splits for, keep the closer ones
-    const int rc = launch_x3(&b, 1, ldb, BT ? X3Fmt::kT : X3Fmt::kN, 0, 0, A, lda, C, ldc, M, K,
-                             beta, false, K % 32 == 0 && t64 >= cus, st);
+    return launch_x3(&b, 1, ldb, BT ? X3Fmt::kT : X3Fmt::kN, 0, 0, A, lda, C, ldc, M, K, beta, must,
+                     K % 32 == 0 && t64 >= cus, st);
+  };
+  if (x3) {
+    const int rc = split_product(false);
     if (rc != 1) return rc;
   }
+  // (a split product without workspace, as in a capture whose warm-up was another
+  // call, goes on here; the kernels below may want even more of it)
+  auto or_whole = [&](int rc) { return x3 && rc == 1 ? split_product(true) : rc; };
   if (M <= 16)
     return launch_mfma_f32<16, 256, 1, 4, BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, batch, beta, st);
   if (M <= 32)
-    return launch_mfma_f32<32, 128, 1, 4, BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, batch, beta, st);
+    return or_whole(launch_mfma_f32<32, 128, 1, 4, BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, batch,
+                                                       beta, st, x3));
   // Tiles (of all the batch's products) covering the chip, K % 32 == 0, 16-byte
   // C rows: the LDS-DMA ring kernel, the whole of K per workgroup.  Two ring slots (plain
   // double buffering) measured fastest: 4, 6, 8 and 10 slots ran 7-27% slower
@@ -635,8 +648,10 @@ int dispatch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, i
     return launch_ring_f32<64, 64, 2, 4, 2, BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K,
                                                 batch, beta, 2, st);
   if (tiles(128, 128) >= cus)
-    return launch_mfma_f32<128, 128, 2, 2, BT, 32>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, batch, beta, st);
-  return launch_mfma_f32<64, 64, 2, 2, BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, batch, beta, st);
+    return or_whole(launch_mfma_f32<128, 128, 2, 2, BT, 32>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K,
+                                                            batch, beta, st, x3));
+  return or_whole(launch_mfma_f32<64, 64, 2, 2, BT>(A, lda, sa, B, ldb, sb, C, ldc, sc, M, N, K, batch,
+                                                    beta, st, x3));
 }
 
 // Batched launch of gemm_t: `batch` products, operand bases `sa`/`sb`/`sc`

@@ -1264,23 +1264,13 @@ int dispatch_padded(const GemmArgs &g, hipStream_t st) {
   if (g.batch != 1 || g.scratch || g.M < 32 || g.K < 128 || g.N < 64 ||
       work < (int64_t(1) << (BNK ? 32 : 29)))
     return 1;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
-    (void)hipGetLastError();  // the launch check must not see it
-    return 1;
-  }
-  if (cs != hipStreamCaptureStatusNone) return 1;  // a graph must not hold the workspace
   const int Kp = (int)cdiv(g.K, 128) * 128;
   const bool pad_a = g.K != Kp || g.lda % 16 != 0 || ((uintptr_t)g.A & 15) != 0;
   const bool pad_b = !BNK || g.K != Kp || g.ldb % 16 != 0 || ((uintptr_t)g.B & 15) != 0;
   const size_t ab = pad_a ? (size_t)g.M * Kp : 0, bb = pad_b ? (size_t)g.N * Kp : 0;
   void *ws = nullptr;
   Workspace lease;
-  if (lease.get(st, ab + bb, &ws, 5) != SIMP_RT_OK) {
-    clear_error();
-    (void)hipGetLastError();
-    return 1;
-  }
+  if (!lease.try_get(st, ab + bb, &ws, 5)) return 1;
   int8_t *a8 = (int8_t *)ws, *b8 = a8 + ab;
   GemmArgs h = g;
   h.K = Kp;

@@ -558,7 +558,7 @@ int pick_splits(int64_t tiles, int steps, int64_t mn, int64_t cus) {
 }
 
 template <int MT, int NT, int NW, int KIND, int PD, bool CARRY = false>
-int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
+int go_x3(X3Args a, bool must, hipStream_t st) {
   const int64_t cus = num_cus(), tm = cdiv(a.M, 16 * MT);
   int64_t tn = 0;
   a.N = 0;
@@ -572,17 +572,10 @@ int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
   int splits = pick_splits(tm * tn, steps, (int64_t)a.M * a.N, cus);
   a.P = nullptr;
   Workspace ws;
-  if (splits > 1) {
-    if (may_split && ws.get(st, sizeof(float) * (size_t)splits * a.M * a.N, (void **)&a.P, 3) != SIMP_RT_OK) {
-      clear_error();
-      (void)hipGetLastError();  // of the allocation: the launch check must not see it
-      may_split = false;
-    }
-    if (!may_split) {
-      if (!must) return 1;
-      splits = 1;
-      a.P = nullptr;
-    }
+  if (splits > 1 && !ws.try_get(st, sizeof(float) * (size_t)splits * a.M * a.N, (void **)&a.P, 3)) {
+    if (!must) return 1;
+    splits = 1;
+    a.P = nullptr;
   }
   a.span = (int)cdiv(steps, splits);
   a.splits = (int)cdiv(steps, a.span);
@@ -604,16 +597,6 @@ int go_x3(X3Args a, bool may_split, bool must, hipStream_t st) {
     SIMP_HIP(hipGetLastError());
   }
   return SIMP_RT_OK;
-}
-
-// Partial sums need the stream's workspace.  A captured call keeps to what it
-// can do without one: a graph must not hold a buffer that a later, larger call
-// may replace.
-bool capturing(hipStream_t st) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();  // the launch check must not see it
-  return true;
 }
 
 }  // namespace
@@ -646,18 +629,17 @@ int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, 
   a.M = M;
   a.K = K;
   a.beta = beta;
-  const bool split = !capturing(st);
 #define X3_GO(MT, NT, NW, ...)                                                         \
-  (fmt == X3Fmt::kN ? go_x3<MT, NT, NW, kBKN, __VA_ARGS__>(a, split, must, st)          \
-                    : go_x3<MT, NT, NW, kBNK, __VA_ARGS__>(a, split, must, st))
+  (fmt == X3Fmt::kN ? go_x3<MT, NT, NW, kBKN, __VA_ARGS__>(a, must, st)                 \
+                    : go_x3<MT, NT, NW, kBNK, __VA_ARGS__>(a, must, st))
   if (fmt == X3Fmt::kW4) {
     // 256 columns on 8 waves, which split A half as often, from 24 tiles on (200x
     // 3200x8640 61 us against 77, 64x3200x32000 60 against 65); fewer leave too
     // few workgroups to a split of K (64x8640x3200 28.8 against 26.8, 64x2048x2048
     // 19 against 15)
 #define X3_W4(MT)                                                          \
-  (cdiv(M, 16 * MT) * cdiv(N, 256) >= 24 ? go_x3<MT, 2, 8, kBW4, 4>(a, split, must, st) \
-                                         : go_x3<MT, 2, 4, kBW4, 4>(a, split, must, st))
+  (cdiv(M, 16 * MT) * cdiv(N, 256) >= 24 ? go_x3<MT, 2, 8, kBW4, 4>(a, must, st) \
+                                         : go_x3<MT, 2, 4, kBW4, 4>(a, must, st))
     return M <= 16 ? X3_W4(1) : M <= 32 ? X3_W4(2) : M <= 64 ? X3_W4(4) : X3_W4(8);
 #undef X3_W4
   }

@@ -107,13 +107,18 @@ WsPool<HipMem> &ws_pool() {
 }
 }  // namespace
 
-int Workspace::get(hipStream_t stream, size_t bytes, void **ptr, int slot) {
+static WsStatus find_workspace(hipStream_t stream, size_t bytes, void **ptr, int slot,
+                               std::unique_lock<std::mutex> &lease) {
   static thread_local char here;  // its address names the thread
   int dev = ensure_device();
-  if (dev < 0) return dev;
-  release();
+  if (dev < 0) return WsStatus::kError;
   const void *thread = stream == hipStreamPerThread ? &here : nullptr;
-  switch (ws_pool().get({dev, stream, thread, slot}, bytes, ptr, lease_)) {
+  return ws_pool().get({dev, stream, thread, slot}, bytes, ptr, lease);
+}
+
+int Workspace::get(hipStream_t stream, size_t bytes, void **ptr, int slot) {
+  release();
+  switch (find_workspace(stream, bytes, ptr, slot, lease_)) {
     case WsStatus::kOk: return SIMP_RT_OK;
     case WsStatus::kCapturing:
       return set_error(SIMP_RT_EUNSUPPORTED,
@@ -123,6 +128,11 @@ int Workspace::get(hipStream_t stream, size_t bytes, void **ptr, int slot) {
       return set_error(SIMP_RT_ENOMEM, "workspace of %zu bytes: out of device memory", bytes);
     default: return SIMP_RT_EHIP;
   }
+}
+
+bool Workspace::try_get(hipStream_t stream, size_t bytes, void **ptr, int slot) {
+  release();
+  return find_workspace(stream, bytes, ptr, slot, lease_) == WsStatus::kOk;
 }
 
 // Looks p up in the registry; returns the device address or nullptr.

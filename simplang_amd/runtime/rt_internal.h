@@ -146,6 +146,9 @@ int num_cus();
 class Workspace {
  public:
   int get(hipStream_t stream, size_t bytes, void **ptr, int slot = 0);
+  // The same for a caller that goes on without: false, and no error raised, when
+  // there is no memory, or no warm-up call left enough for a captured one.
+  bool try_get(hipStream_t stream, size_t bytes, void **ptr, int slot);
   void release() {
     if (lease_.owns_lock()) lease_.unlock();
   }
@@ -222,7 +225,7 @@ int launch_w4d8(const W4D8Args &a, hipStream_t st);
 // symmetric W4 rows [n, K/2] with scales [n, lds].  Any alignment and leading
 // dimension; W4: K and gs multiples of 32, rows of W 4-byte aligned.  Returns 1
 // when it does not serve the shape, and, unless `must`, when it wants K splits
-// and their workspace cannot be had.  `carry` (fp32): sums may be carried
+// and their workspace cannot be had (a captured call: its warm-up left none).  `carry` (fp32): sums may be carried
 // through the whole of K in the MFMA accumulator, faster and as exact as the
 // fp32 MFMA kernels' over as long a K; else they are several times more exact.
 enum class X3Fmt { kN, kT, kW4 };
