@@ -1209,14 +1209,14 @@ int capture_step(LlamaModel &m, int mode) {
 }
 
 // Runs the first n tokens of the prompt (already on the device) as rows of
-// matrices; *done receives how many of them it took, n or 0 (shapes that the
-// row kernels do not take, no memory for the activations, or too few tokens:
-// a pass costs about as much as five steps: 110M 1.4 ms for 199 tokens, 3B W4
+// matrices; *done receives how many of them it took, n or 0 (shapes or weights
+// that the row kernels do not take, no memory for the activations, or too few
+// tokens: the steps then take the prompt, writing every cache row again; a pass costs about as much as five steps: 110M 1.4 ms for 199 tokens, 3B W4
 // 4.4 ms for 31, against 0.31 and 0.88 ms a step).
 constexpr int64_t kPrefillMin = 8, kPrefillRows = 512;
 int prefill_prompt(LlamaModel &m, int64_t n, int64_t *done) {
   *done = 0;
-  if (n < kPrefillMin || !prefill_supported(m.cfg, m.hs)) return SIMP_RT_OK;
+  if (n < kPrefillMin || !prefill_supported(m.cfg, m.w, m.hs)) return SIMP_RT_OK;
   if (!m.pre_ws) {
     const int rows = (int)std::min<int64_t>(kPrefillRows, m.cfg.seq_len);
     if (hipMalloc(&m.pre_ws, sizeof(float) * prefill_floats(m.cfg, rows)) != hipSuccess) {
@@ -1229,6 +1229,7 @@ int prefill_prompt(LlamaModel &m, int64_t n, int64_t *done) {
   const PrefillArgs a{&m.cfg, &m.w, m.kv_dim, m.hs, m.prompt, m.kcache, m.vcache, m.rope,
                       m.pre_ws, m.pre_rows};
   const int rc = prefill(a, n, m.stream);
+  if (rc == 1) return SIMP_RT_OK;
   if (rc == SIMP_RT_OK) *done = n;
   return rc;
 }

@@ -212,12 +212,15 @@ __global__ void __launch_bounds__(256)
 
 }  // namespace
 
-bool prefill_supported(const simp_rt_llama_config &c, int hs) {
+bool prefill_supported(const simp_rt_llama_config &c, const simp_rt_llama_weights &w, int hs) {
   const int64_t kv = (int64_t)hs * c.n_kv_heads;
   // float4 rows of a head, in the attention kernel's registers
   if (hs % 4 != 0 || hs > 128 || c.dim % 4 != 0 || kv % 4 != 0 || c.hidden_dim > INT32_MAX / 2) return false;
-  return c.weight_format != SIMP_RT_W_W4S ||
-         (c.dim % 32 == 0 && c.hidden_dim % 32 == 0 && c.group_size % 32 == 0);
+  if (c.weight_format != SIMP_RT_W_W4S) return true;
+  // 4-byte loads of W4 rows, which are whole 16 bytes apart
+  for (const void *p : {w.q_wq, w.q_wk, w.q_wv, w.q_wo, w.q_w1, w.q_w2, w.q_w3})
+    if (((uintptr_t)p & 3) != 0) return false;
+  return c.dim % 32 == 0 && c.hidden_dim % 32 == 0 && c.group_size % 32 == 0;
 }
 
 size_t prefill_floats(const simp_rt_llama_config &c, int rows) {

@@ -251,8 +251,9 @@ struct PrefillArgs {
   float *ws;              // prefill_floats(cfg, rows) floats
   int rows;               // tokens per pass
 };
-bool prefill_supported(const simp_rt_llama_config &cfg, int hs);
+bool prefill_supported(const simp_rt_llama_config &cfg, const simp_rt_llama_weights &w, int hs);
 size_t prefill_floats(const simp_rt_llama_config &cfg, int rows);
+// SIMP_RT_OK, an error, or 1 where a product is not served.
 int prefill(const PrefillArgs &a, int64_t n_tokens, hipStream_t st);
 // C = beta*C + A*B (beta 0 or 1), row-major with leading dimensions in elements.
 int launch_matmul_f32(const float *A, int64_t lda, const float *B, int64_t ldb, float *C,

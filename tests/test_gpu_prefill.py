@@ -59,6 +59,32 @@ def test_prompt_equals_steps(dev, cfg, n):
     b.close()
 
 
+@pytest.mark.parametrize("off", [1, 2, 4, 8])
+def test_prompt_with_unaligned_w4_weights(dev, off):
+    """W4 matrices that start at any byte: the steps take the prompt where the
+    row products (4-byte loads) cannot, and generation is the same."""
+    import torch
+    cfg = _cfg(weight_format=1)
+    w = make_model(cfg, dev, seed=5)
+    moved = dict(w)
+    for k in w:
+        if k.startswith("q_w"):
+            buf = torch.empty(w[k].numel() + 16, dtype=torch.uint8, device=dev)
+            moved[k] = buf[off:off + w[k].numel()]
+            moved[k].copy_(w[k].reshape(-1).view(torch.uint8))
+            assert moved[k].data_ptr() % 16 == off
+    prompt = np.arange(20, dtype=np.int32)
+    a, b = sa.Llama(cfg, w), sa.Llama(cfg, moved)
+    la, lb = (torch.empty(cfg["vocab_size"], device=dev) for _ in range(2))
+    want, got = a.generate(prompt, 6), b.generate(prompt, 6)
+    a.forward(int(want[-1]), len(want) - 1, la)
+    b.forward(int(want[-1]), len(want) - 1, lb)
+    a.close()
+    b.close()
+    assert np.array_equal(got, want)
+    assert float((la - lb).abs().max()) <= 2e-5 * float(la.abs().max())
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 def test_prompt_against_oracle(dev, orc, fmt):
     """Greedy tokens and the next logits after a 60-token prompt."""
