@@ -472,6 +472,9 @@ constexpr int kColsumRows = 1;  // the kernel's MFMAs; tiles grouped by tile row
                                 // workgroup forms the sums for every tile
 constexpr int kColsumOnce = 2;  // the kernel's MFMAs; tiles grouped by tile columns, so a
                                 // workgroup forms them once per column tile it visits
+// its stores of C: rows of any alignment and N, 16-byte aligned rows, and rows on
+// 64 bytes (whole half lines, streamed past L2)
+constexpr int kStoreAny = 0, kStore16 = 1, kStoreStream = 2;
 template <int STAGES, bool AU8, bool BNK, int CSM = kColsumPass>
 __global__ void __launch_bounds__(512)
     gemm_i8_dma(const int8_t *__restrict__ A, int64_t lda, const int8_t *__restrict__ B,
@@ -671,7 +674,9 @@ __global__ void __launch_bounds__(512)
         if (row >= M || col >= N) continue;
         const v4i v = acc[i][j] + bias;
         int32_t *dst = C + (int64_t)row * ldc + col;
-        if (vec_store) {
+        if (vec_store == kStore16) {
+          *(v4i *)dst = v;
+        } else if (vec_store == kStoreStream) {
           // streaming store: C is not re-read here, and the all-CU store burst
           // at a tile's end drains faster without allocating in L2 (measured
           // 4-5% on the whole kernel at 8192^3)
@@ -1339,12 +1344,38 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     SIMP_HIP(hipGetLastError());
     return SIMP_RT_OK;
   }
-  // (the kernels for B_T read whole rows and take any N: column by column
-  // stores where a row of C does not end with a 16-byte one)
-  const bool any_n = BNK && g.K % 128 == 0;
-  if (g.batch == 1 && tiles(256, 256) >= cus && (any_n || g.N % 16 == 0)) {
+  // N % 16 != 0 with B_T: the kernels below read whole rows of B_T and take any
+  // N (column by column stores where a row of C does not end with 16 bytes).
+  // dispatch_tiles runs two 128x128 workgroups per CU and splits K; against it
+  // they are ahead only where their own rounds over the CUs are well filled and
+  // K is long enough (kernel time at 3600 sizes M x N x K, us, dispatch_tiles /
+  // these, column sums in the kernel either way):
+  //   256x256: rounds three quarters full from K = 2048 (8192x3204x2048 92 / 79),
+  //     five eighths from 4096 (4096x5001x4096 129 / 120), any from 8192; with
+  //     shorter K the tiles' fill and drain show (4096x4100x256 22 / 36)
+  //   128x128: one round or three, for which the two-per-CU tiles take one and two
+  //     of twice the length (1024x3204x4096 34 / 26), not two (2048x2052x4096 41 /
+  //     45); 1500x1300x512, on half of the CUs, 10% slower
+  //   64x64: one round (dispatch_tiles splits K: a zero fill and atomics;
+  //     512x1028x1024 21 / 5.0), not two (1024x1028x1024 7.5 / 8.5); u8 with long K
+  //     not where rows are padding (200x2500x8192 24 / 25)
+  const int64_t t256 = tiles(256, 256), t128 = tiles(128, 128), t64 = tiles(64, 64);
+  const bool n16 = g.N % 16 == 0, any_n = BNK && g.K % 128 == 0;
+  const int64_t room = cdiv(t256, cus) * cus;  // of the 256x256 tiles' rounds
+  const bool ok256 = n16 || (any_n && (g.K >= 8192 || (g.K >= 4096 && 8 * t256 >= 5 * room) ||
+                                       (g.K >= 2048 && 4 * t256 >= 3 * room)));
+  const bool ok128 = n16 || (any_n && ((cdiv(t128, cus) % 2 == 1 && ((4 * t128 >= 3 * cus && g.K >= 1024) ||
+                                                                     (2 * t128 >= cus && g.K >= 3072))) ||
+                                       (t128 <= cus && g.K >= 8192)));
+  const bool ok64 = n16 || (any_n && t64 <= cus &&
+                            (!AU8 || g.K < 8192 || 8 * (int64_t)g.M >= 7 * 64 * cdiv(g.M, 64)));
+  if (g.batch == 1 && t256 >= cus && ok256) {
     const int tm = (int)cdiv(g.M, 256), tn = (int)cdiv(g.N, 256);
-    const int vec = g.N % 4 == 0 && g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
+    // streaming stores only into rows that start on 64 bytes: partial lines that
+    // bypass L2 ran 8192x8196x256 at 268 us against 98
+    const int vec = g.N % 4 != 0 || g.ldc % 4 != 0 || ((uintptr_t)g.C & 15) != 0 ? kStoreAny
+                    : g.ldc % 16 == 0 && ((uintptr_t)g.C & 63) == 0           ? kStoreStream
+                                                                              : kStore16;
     // persistent grid: one workgroup per CU, a multiple of 8 (XCD round-robin)
     const int grid = (int)std::max<int64_t>(8, std::min<int64_t>(cus, (int64_t)tm * tn) / 8 * 8);
     // B[K,N] with 16-byte aligned rows is read in place by gemm_i8_dma
@@ -1449,8 +1480,8 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     // A deeper prefetch spreads an XCD's CUs over more operand lines than its
     // L2 keeps; a shallower one exposes the load latency when a CU has the
     // memory system to itself for longer (long K, part of the chip idle).
-    const bool ok = g.batch == 1 && g.K % 128 == 0 && (any_n || g.N % 16 == 0) && g.ldb % 16 == 0 &&
-                    ((uintptr_t)g.B & 15) == 0;
+    const bool ok = g.batch == 1 && g.K % 128 == 0 && g.ldb % 16 == 0 && ((uintptr_t)g.B & 15) == 0 &&
+                    t256 < cus;
     const int vec = g.N % 4 == 0 && g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
     auto ring = [&](auto bm, auto slots) {
       constexpr int BM = decltype(bm)::value, SL = decltype(slots)::value;
@@ -1470,12 +1501,11 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     // CUs and K is long (96 and 128 x 3200 x 8640: 20.2 and 21.4 us on 68
     // tiles against 22.4 and 22.7 on 270); 4 slots where the operands stream
     // from HBM rather than L2 (128x3200x32000: 24.5 against 25.0 us).
-    const int64_t t128 = tiles(128, 128), t64 = tiles(64, 64);
-    if (ok && g.M > 64 && (2 * t128 >= cus || (t64 > cus && 4 * t128 >= cus && g.K >= 3072))) {
+    if (ok && ok128 && g.M > 64 && (2 * t128 >= cus || (t64 > cus && 4 * t128 >= cus && g.K >= 3072))) {
       if ((int64_t)g.K * (g.M + g.N) >= (int64_t(64) << 20)) return ring(I128(), I4());
       return ring(I128(), I2());
     }
-    if (ok && 2 * t64 >= cus && g.M > 32) {
+    if (ok && ok64 && 2 * t64 >= cus && g.M > 32) {
       if (t64 <= cus && (g.K <= 2048 || (g.K <= 4096 && 4 * t64 >= 3 * cus)))
         return ring(I64(), I2());
       return ring(I64(), I4());

@@ -48,3 +48,29 @@ def test_any_batch(dev):
     c = torch.empty(5, 37, 45, dtype=torch.int32, device=dev)
     sa.tensor_batch_matmul(torch.from_numpy(a).to(dev), torch.from_numpy(b).to(dev), c)
     assert np.array_equal(c.cpu().numpy(), (a.astype(np.float64) @ b.astype(np.float64)).astype(np.int32))
+
+
+# B_T with K % 128 == 0 and N % 16 != 0, C of any pitch: tiles with and without K
+# splits, one round of 64x64 and 128x128 and two, 256x256 streamed and not
+NT = [(100, 260, 256, 0), (512, 1028, 1024, 0), (1024, 1028, 1024, 4), (1024, 3205, 3072, 0),
+      (2048, 2052, 1024, 1), (2050, 4100, 8192, 0), (4096, 8196, 256, 0), (4100, 5001, 4096, 3),
+      (4096, 8192, 2048, 16), (4096, 8192, 2048, 4)]
+
+
+@pytest.mark.parametrize("u8", [False, True])
+@pytest.mark.parametrize("M,N,K,pad", NT)
+def test_nt_columns(dev, M, N, K, pad, u8):
+    import torch
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a = torch.randint(0, 256, (M, K), dtype=torch.uint8, device=dev, generator=g)
+    b = torch.randint(-128, 128, (N, K), dtype=torch.int8, device=dev, generator=g)
+    a = a if u8 else a.view(torch.int8)
+    c = torch.full((M + 1, N + pad), 9, dtype=torch.int32, device=dev)
+    (sa.matmul_nt_u8s8_i32 if u8 else sa.tensor_matmul_nt_i8)(a, b, c[:M, :N])
+    rows = torch.tensor([0, 1, M // 2, M - 65, M - 1], device=dev)
+    cols = torch.tensor([0, 15, N // 2, N - 17, N - 4, N - 1], device=dev)
+    bd = b.double().t().contiguous()
+    assert torch.equal(c[rows, :N], (a[rows].double() @ bd).int())
+    assert torch.equal(c[:M, cols], (a.double() @ bd[:, cols].contiguous()).int())
+    assert bool((c[M] == 9).all()) and bool((c[:, N:] == 9).all())
