@@ -1258,24 +1258,43 @@ int dispatch(const GemmArgs &g, hipStream_t st);
 // Products that the aligned kernels cannot read, large enough to pay for copies
 // of their operands with rows of a multiple of 128 bytes (B transposed on the
 // way): the kernels for B_T then run at their full rate.  Returns 1 where the
-// copies do not pay or their workspace cannot be had.
-//   B[K,N], from 2^29 products on: 717x2051x1533 18 us against 38 on the
-//   byte-aligned tiles (their loads are 4 bytes wide), 4095x4097x4099 110
-//   against 600, 1000^3 18 against 25.  B_T, from 2^32: 2000x5000x3001 70 us
-//   against 166, while 717x2051x1533 stays at 17 either way.
+// copies do not pay or their workspace cannot be had.  Kernel time of all three
+// launches against the byte-aligned tiles, M x N x K, us:
+//   B[K,N] (the tiles' loads are 4 bytes wide), from 2^29 products on:
+//     * the kernel behind the copies has a tile for half of the CUs (it needs that
+//       to leave dispatch_tiles) and 80 rows or more share the copy of B:
+//       160x3001x1001 14 against 24, 717x2051x1533 21 against 39, 2047x4097x4099
+//       93 against 401; below, the copies come on top of much the same tiles:
+//       128x3001x1001 23 against 18, 320x1533x1535 23 against 20
+//     * or B is 24 MB and larger, from which on the tiles' own reads of it are
+//       what takes the time: 33x3201x8639 29 against 38
+//       (48x4097x4099 27 against 22)
+//     * or K is long, from 192 rows on: 256x1001x8191 35 against 41
+//       (320x1001x3001 27 against 24)
+//   B_T, from 9 * 2^29 products and 160 rows on (192x8639x3201 36 against 44), or
+//     65 where 64x64 tiles would come in two rounds or less (96x8639x8639 74
+//     against 103); fewer rows read B faster where it lies (96x31999x3199 59
+//     against 52, 64x8639x8639 52 against 40)
+// Copies of more than 4 GiB are not made (the buffer stays with the stream).
 template <bool BNK, bool AU8>
 int dispatch_padded(const GemmArgs &g, hipStream_t st) {
   const int64_t work = (int64_t)g.M * g.N * g.K;
-  if (g.batch != 1 || g.scratch || g.M < 32 || g.K < 128 || g.N < 64 ||
-      work < (int64_t(1) << (BNK ? 32 : 29)))
-    return 1;
+  if (g.batch != 1 || g.scratch || g.M < 32 || g.K < 128 || g.N < 64) return 1;
+  const int64_t cus = num_cus(), t64 = cdiv(g.M, 64) * cdiv(g.N, 64);
+  const bool pays =
+      BNK ? work >= 9 * (int64_t(1) << 29) && (g.M >= 160 || (g.M > 64 && t64 <= 2 * cus))
+          : work >= (int64_t(1) << 29) &&
+                ((g.M >= 80 && 2 * t64 >= cus) || (int64_t)g.N * g.K >= 24000000 ||
+                 (g.M >= 192 && g.K > 6144));
+  // (a grid's y has 65535 blocks, of 128 k-rows of B each)
+  if (!pays || cdiv(g.K, 128) > 65535) return 1;
   const int Kp = (int)cdiv(g.K, 128) * 128;
   const bool pad_a = g.K != Kp || g.lda % 16 != 0 || ((uintptr_t)g.A & 15) != 0;
   const bool pad_b = !BNK || g.K != Kp || g.ldb % 16 != 0 || ((uintptr_t)g.B & 15) != 0;
   const size_t ab = pad_a ? (size_t)g.M * Kp : 0, bb = pad_b ? (size_t)g.N * Kp : 0;
   void *ws = nullptr;
   Workspace lease;
-  if (!lease.try_get(st, ab + bb, &ws, 5)) return 1;
+  if (ab + bb > (size_t(4) << 30) || !lease.try_get(st, ab + bb, &ws, 5)) return 1;
   int8_t *a8 = (int8_t *)ws, *b8 = a8 + ab;
   GemmArgs h = g;
   h.K = Kp;

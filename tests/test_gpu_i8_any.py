@@ -40,6 +40,34 @@ def test_any_size_and_alignment(dev, M, N, K, nt, u8):
         assert (got[M] == 9).all() and (got[:, N] == 9).all()
 
 
+# both sides of the lines between padded copies and byte-aligned tiles (rows, tiles,
+# size of B, K, products), and more k-rows than a grid of copies has blocks for
+PADDED = [(79, 8191, 1001), (80, 8191, 1001), (128, 3001, 1401), (160, 3001, 1401), (33, 3199, 8639),
+          (33, 2699, 8639), (191, 1001, 6145), (192, 1001, 6145), (160, 6001, 5101), (64, 9001, 9001),
+          (65, 9001, 9001), (32, 64, 8390001)]
+
+
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("M,N,K", PADDED)
+def test_padded_or_not(dev, M, N, K, nt):
+    import torch
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    small = K > 1 << 20  # sums below 2^31
+    a = torch.randint(-2 if small else -128, 3 if small else 128, (M, K), dtype=torch.int8, device=dev,
+                      generator=g)
+    b = torch.randint(-2 if small else -128, 3 if small else 128, (N, K) if nt else (K, N),
+                      dtype=torch.int8, device=dev, generator=g)
+    c = torch.empty((M, N), dtype=torch.int32, device=dev)
+    (sa.tensor_matmul_nt_i8 if nt else sa.tensor_matmul_i8)(a, b, c)
+    step = 1 << 20
+    want = torch.zeros((M, N), dtype=torch.float64, device=dev)
+    for k in range(0, K, step):
+        bk = b[:, k:k + step].double().t().contiguous() if nt else b[k:k + step].double()
+        want += a[:, k:k + step].double() @ bk
+    assert torch.equal(c, want.int())
+
+
 def test_any_batch(dev):
     import torch
     rng = np.random.default_rng(1)
