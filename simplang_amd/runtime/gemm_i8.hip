@@ -144,8 +144,10 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
       if (A_TOT % NT == 0 || c < A_TOT) {
         const int kc = c % KC, m = c / KC;
         const int gm = m0 + m, gk = k0 + kc * 16;
-        if (gm < M && gk < kend)
-          v = ANY ? row16_any(A + (int64_t)gm * lda, gk, K) : *(const uint4 *)(A + (int64_t)gm * lda + gk);
+        if (gm < M && gk < kend) {
+          if constexpr (ANY) v = row16_any(A + (int64_t)gm * lda, gk, K);
+          else v = *(const uint4 *)(A + (int64_t)gm * lda + gk);
+        }
       }
       ra[i] = v;
     }
@@ -157,8 +159,10 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
         if (B_TOT % NT == 0 || c < B_TOT) {
           const int kc = c % KC, n = c / KC;
           const int gn = n0 + n, gk = k0 + kc * 16;
-          if (gn < N && gk < kend)
-            v = ANY ? row16_any(B + (int64_t)gn * ldb, gk, K) : *(const uint4 *)(B + (int64_t)gn * ldb + gk);
+          if (gn < N && gk < kend) {
+            if constexpr (ANY) v = row16_any(B + (int64_t)gn * ldb, gk, K);
+            else v = *(const uint4 *)(B + (int64_t)gn * ldb + gk);
+          }
         }
         rbq[i] = v;
       }
@@ -174,10 +178,9 @@ __global__ void __launch_bounds__(WGM *WGN * 64)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int gk = k0 + kq * 16 + r;
-          rbd[i][r] = 0u;
-          if (on && gn < N && gk < kend)
-            rbd[i][r] = ANY ? *(const u1any *)(p + (int64_t)r * ldb) >> (8 * back)
-                            : *(const uint32_t *)(p + (int64_t)r * ldb);
+          const bool in = on && gn < N && gk < kend;
+          if constexpr (ANY) rbd[i][r] = in ? *(const u1any *)(p + (int64_t)r * ldb) >> (8 * back) : 0u;
+          else rbd[i][r] = in ? *(const uint32_t *)(p + (int64_t)r * ldb) : 0u;
         }
       }
     }
@@ -472,14 +475,11 @@ constexpr int kColsumRows = 1;  // the kernel's MFMAs; tiles grouped by tile row
                                 // workgroup forms the sums for every tile
 constexpr int kColsumOnce = 2;  // the kernel's MFMAs; tiles grouped by tile columns, so a
                                 // workgroup forms them once per column tile it visits
-// its stores of C: rows of any alignment and N, 16-byte aligned rows, and rows on
-// 64 bytes (whole half lines, streamed past L2)
-constexpr int kStoreAny = 0, kStore16 = 1, kStoreStream = 2;
 template <int STAGES, bool AU8, bool BNK, int CSM = kColsumPass>
 __global__ void __launch_bounds__(512)
     gemm_i8_dma(const int8_t *__restrict__ A, int64_t lda, const int8_t *__restrict__ B,
                 int64_t ldb, int32_t *__restrict__ C, int64_t ldc, int M, int N, int K,
-                int tiles_m, int tiles_n, const int32_t *__restrict__ colsum, int vec_store) {
+                int tiles_m, int tiles_n, const int32_t *__restrict__ colsum, int stream) {
   constexpr int BM = 256, BN = 256, BK = 64, WGN = 4;
   constexpr int WM = 128, WN = 64, FM = WM / 16, FN = WN / 16;
   constexpr int STAGE = (BM + BN) * BK;  // bytes
@@ -674,9 +674,7 @@ __global__ void __launch_bounds__(512)
         if (row >= M || col >= N) continue;
         const v4i v = acc[i][j] + bias;
         int32_t *dst = C + (int64_t)row * ldc + col;
-        if (vec_store == kStore16) {
-          *(v4i *)dst = v;
-        } else if (vec_store == kStoreStream) {
+        if (stream) {
           // streaming store: C is not re-read here, and the all-CU store burst
           // at a tile's end drains faster without allocating in L2 (measured
           // 4-5% on the whole kernel at 8192^3)
@@ -1392,9 +1390,7 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     const int tm = (int)cdiv(g.M, 256), tn = (int)cdiv(g.N, 256);
     // streaming stores only into rows that start on 64 bytes: partial lines that
     // bypass L2 ran 8192x8196x256 at 268 us against 98
-    const int vec = g.N % 4 != 0 || g.ldc % 4 != 0 || ((uintptr_t)g.C & 15) != 0 ? kStoreAny
-                    : g.ldc % 16 == 0 && ((uintptr_t)g.C & 63) == 0           ? kStoreStream
-                                                                              : kStore16;
+    const int stream = g.N % 4 == 0 && g.ldc % 16 == 0 && ((uintptr_t)g.C & 63) == 0;
     // persistent grid: one workgroup per CU, a multiple of 8 (XCD round-robin)
     const int grid = (int)std::max<int64_t>(8, std::min<int64_t>(cus, (int64_t)tm * tn) / 8 * 8);
     // B[K,N] with 16-byte aligned rows is read in place by gemm_i8_dma
@@ -1436,7 +1432,7 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
       auto launch = [&](auto bnk, auto csm) {
         hipLaunchKernelGGL((gemm_i8_dma<4, AU8, decltype(bnk)::value, decltype(csm)::value>),
                            dim3(grid), dim3(512), 0, st, g.A, g.lda, g.B, g.ldb, g.C, g.ldc, g.M,
-                           g.N, g.K, tm, tn, (const int32_t *)nullptr, vec);
+                           g.N, g.K, tm, tn, (const int32_t *)nullptr, stream);
       };
       using Rows = std::integral_constant<int, kColsumRows>;
       using Once = std::integral_constant<int, kColsumOnce>;
@@ -1474,7 +1470,7 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
       KernelTimer kt(st, "gemm_i8_dma");
       hipLaunchKernelGGL((gemm_i8_dma<4, AU8, true>), dim3(grid), dim3(512), 0, st, h.A, h.lda,
                          h.B, h.ldb, h.C, h.ldc, h.M, h.N, h.K, tm, tn, (const int32_t *)colsum,
-                         vec);
+                         stream);
     } else {
       KernelTimer kt(st, "gemm_i8_nt16");
       hipLaunchKernelGGL((gemm_i8_nt16<256, 256, 128, 2, 4, AU8>), dim3(tm * tn), dim3(512), 0,
