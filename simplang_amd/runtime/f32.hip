@@ -503,6 +503,18 @@ __global__ void __launch_bounds__(256)
   *o = beta != 0.f ? *o + v : v;
 }
 
+// K splits of launch_mfma_f32, in steps of 16: until there are about four blocks
+// per CU, each split at least 64 deep, the partials no larger than the operands
+// (they are written and read once more) and within 1 GiB.
+int64_t mfma_splits(int64_t cus, int64_t tiles, int M, int N, int K, int64_t batch) {
+  const int64_t mn = (int64_t)M * N, ops = (int64_t)M * K + (int64_t)K * N;
+  if (tiles * batch >= 4 * cus || K < 512) return 1;
+  int64_t splits = std::min<int64_t>(std::min<int64_t>(cdiv(4 * cus, tiles * batch), 32), cdiv(K, 16) / 4);
+  splits = std::min<int64_t>(splits, ops / std::max<int64_t>(mn, 1));
+  while (splits > 1 && batch * splits * mn * 4 > (int64_t(1) << 30)) splits--;
+  return std::max<int64_t>(splits, 1);
+}
+
 // or_one: 1 instead of an error when there is no workspace for the K splits.
 template <int BM, int BN, int WGM, int WGN, bool BT, int BK = 16>
 int launch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, int64_t ldb,
@@ -512,18 +524,8 @@ int launch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, int
   if (tiles > INT32_MAX)
     return set_error(SIMP_RT_EUNSUPPORTED, "gemm: %lld output tiles exceed one launch",
                      (long long)tiles);
-  // split K until there are about four blocks per CU: each split at least 64
-  // deep, the partials no larger than the operands (they are written and read
-  // once more) and within 1 GiB
-  const int64_t cus = num_cus(), nkt = cdiv(K, 16);
-  int64_t splits = 1;
-  if (tiles * batch < 4 * cus && K >= 512) {
-    const int64_t mn = (int64_t)M * N, ops = (int64_t)M * K + (int64_t)K * N;
-    splits = std::min<int64_t>(std::min<int64_t>(cdiv(4 * cus, tiles * batch), 32), nkt / 4);
-    splits = std::min<int64_t>(splits, ops / std::max<int64_t>(mn, 1));
-    while (splits > 1 && (int64_t)batch * splits * mn * 4 > (int64_t(1) << 30)) splits--;
-    splits = std::max<int64_t>(splits, 1);
-  }
+  const int64_t nkt = cdiv(K, 16);
+  int64_t splits = mfma_splits(num_cus(), tiles, M, N, K, batch);
   const int k_span = (int)(cdiv(nkt, splits) * 16);
   splits = cdiv(K, k_span);
   float *P = nullptr;
@@ -577,6 +579,35 @@ int launch_ring_f32(const float *A, int64_t lda, int64_t sa, const float *B, int
   return SIMP_RT_OK;
 }
 
+// The time in us that dispatch_mfma_f32's own kernels take for one product of
+// more than 16 rows, for comparison with split_f32_us (gemm_x3.hip): rounds of
+// tiles over the CUs times K steps, the traffic of partial sums and of C.  Fitted
+// to 9000 sizes (M 17 to 4096, N 4 to 8192, K 16 to 8640, B[K,N] and B_T), which
+// it meets to 6% in the root mean square; choosing by the two costs 0.2% of the
+// time on average against the better of the two.  (The split products everywhere
+// but below about a MB of weights, the rule before, cost 3%, and 18 to 80% at
+// 128x1024x512 (M x N x K) with B_T, 64x768x768 and 4096x4096x48.)
+double mfma_f32_us(int64_t cus, int M, int N, int K) {
+  auto tiles = [&](int bm, int bn) { return cdiv(M, bm) * cdiv(N, bn); };
+  const double mn = 1e-6 * M * N, steps = K / 32.;
+  auto rounds = [&](int bm, int bn) { return (double)cdiv(tiles(bm, bn), cus); };
+  if (M > 32 && K % 32 == 0) {  // gemm_f32_ring
+    if (K <= 256 && tiles(64, 64) >= cus) return 3.2 + rounds(64, 64) * (0.54 * steps + 0.45) + 0.26 * mn;
+    if (tiles(256, 128) >= 2 * cus) return 7.4 + rounds(256, 128) * 3.9 * steps + 0.6 * mn;
+    if (tiles(128, 128) >= cus) return 5.6 + rounds(128, 128) * (2.03 * steps + 0.22) + 0.64 * mn;
+    if (tiles(64, 64) >= cus) return 4.2 + rounds(64, 64) * 0.565 * steps;
+  }
+  const bool t128 = M > 32 && tiles(128, 128) >= cus;
+  const int64_t t = M <= 32 ? tiles(32, 128) : t128 ? tiles(128, 128) : tiles(64, 64);
+  const int64_t span = cdiv(cdiv(K, 16), mfma_splits(cus, t, M, N, K, 1)), s = cdiv(K, 16 * span);
+  const double blocks = (double)(t * s) / (double)cus;  // per CU, several at a time
+  if (M <= 32)
+    return 2.8 + 0.535 * span + blocks * (0.09 * span + 0.95) + (s > 1 ? 2.45 + 1.67 * (s + 1) * mn : 0.);
+  if (!t128)
+    return 3.1 + 0.437 * span + blocks * (0.18 * span + 0.3) + (s > 1 ? 2.1 + 1.9 * (s + 1) * mn : 0.);
+  return 6.4 + 1.13 * (double)cdiv(t * s, cus) * span + 0.77 * mn + (s > 1 ? 10.4 + 0.47 * (s + 1) * mn : 0.);
+}
+
 // fp32 GEMM dispatch on the MFMA path (returns 1 when the operands do not meet
 // its requirements, for the caller's SIMT fallback).
 template <bool BT>
@@ -589,22 +620,15 @@ int dispatch_mfma_f32(const float *A, int64_t lda, int64_t sa, const float *B, i
   if (!ok) return 1;
   const int64_t cus = num_cus();
   auto tiles = [&](int bm, int bn) { return cdiv(M, bm) * cdiv(N, bn) * batch; };
-  // one round of 64x64 ring tiles with a short K stays ahead of the split
-  // products' larger tiles (200x256x4096 8.3 us against 9.7, 512x768x2048 18.4
-  // against 19.6; 300x256x4096 12.9 against 9.9, 512x2048x2048 43 against 32)
   const int64_t t64 = tiles(64, 64);
-  const bool one_round = K % 32 == 0 && K <= 1024 && t64 >= cus && 8 * t64 <= 9 * cus;
-  // products of about a MB of weights likewise (two launches either way):
-  // 24x768x768 9.2 us against 9.8, 128x768x768 with B_T 10.5 against 11.4
-  const int64_t kn = (int64_t)K * N;
-  const bool small = M <= 32 ? kn < (1 << 20) : BT && M <= 128 && kn <= (5 << 18);
-  const bool x3 = batch == 1 && M > 16 && !one_round && !small;
+  // carried sums where the ring kernel would carry its own through all of K; the
+  // smaller shapes, whose K it splits for, keep the closer ones
+  const bool carry = K % 32 == 0 && t64 >= cus;
+  const bool x3 = batch == 1 && M > 16 && split_f32_us(cus, BT, M, N, K, carry) < mfma_f32_us(cus, M, N, K);
   auto split_product = [&](bool must) {
     const X3Mat b{B, nullptr, N};
-    // carried sums where the ring kernel would carry its own through all of K;
-    // the smaller shapes, whose K it splits for, keep the closer ones
     return launch_x3(&b, 1, ldb, BT ? X3Fmt::kT : X3Fmt::kN, 0, 0, A, lda, C, ldc, M, K, beta, must,
-                     K % 32 == 0 && t64 >= cus, st);
+                     carry, st);
   };
   if (x3) {
     const int rc = split_product(false);

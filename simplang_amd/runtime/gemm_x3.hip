@@ -542,19 +542,26 @@ __global__ void __launch_bounds__(256)
 // partial sums cost a launch (about three steps' time) and their traffic (a
 // step is about 1 us, in which 4 MB go by).  Measured (W4, 200 x 3200 -> 8640,
 // 68 tiles: 3 / 6 / 7 splits 61 / 72 / 71 us; fp32 128 x 2048 x 8192,
-// 128 tiles: 1 / 2 / 4 splits 70 / 39 / 39 us).
+// 128 tiles: 1 / 2 / 4 splits 70 / 39 / 39 us).  More than 16 splits only within
+// one round (64x256x8640, 2 tiles: 16 / 30 splits 19.7 / 14.8 us).
 int pick_splits(int64_t tiles, int steps, int64_t mn, int64_t cus) {
   int best = 1;
   double cost = 0;
-  for (int s = 1; s <= 16 && s * 4 <= std::max(steps, 4); s++) {
+  for (int s = 1; s <= 32 && s * 4 <= std::max(steps, 4); s++) {
     const int span = (int)cdiv(steps, s);
     if (cdiv(steps, span) != s) continue;
+    if (s > 16 && tiles * s > cus) break;
     if (s > 1 && s * mn > (int64_t(1) << 28)) break;  // 1 GiB of partials
     const double c = (double)cdiv(tiles * s, cus) * (span + 4) +
                      (s > 1 ? 3.0 + 1e-6 * (double)(s + 1) * (double)mn : 0.0);
     if (s == 1 || c < cost) best = s, cost = c;
   }
   return best;
+}
+
+// 128x256 tiles from two per CU on (4096^3: 686 us against 790 with 64x128)
+bool large_tiles(int64_t cus, int M, int64_t N, bool carry) {
+  return M > 32 && carry && cdiv(M, 128) * cdiv(N, 256) >= 2 * cus;
 }
 
 template <int MT, int NT, int NW, int KIND, int PD, bool CARRY = false>
@@ -600,6 +607,30 @@ int go_x3(X3Args a, bool must, hipStream_t st) {
 }
 
 }  // namespace
+
+// The model behind pick_splits with the constants of each tile in us, fitted
+// together with mfma_f32_us (f32.hip), which tells the sizes and what choosing by
+// it costs: fixed and per K split, per K step and round of tiles, and per million
+// partial sums and outputs.
+double split_f32_us(int64_t cus, bool bt, int M, int N, int K, bool carry) {
+  struct Cost { double fixed, split, step, round, part, out; };
+  static const Cost k32[2] = {{3.25, 2.0, 0.70, 0, 2.2, 0.5}, {3.8, 2.2, 0.60, 0, 2.5, 2.6}},
+                    k64[2] = {{1.3, 2.0, 0.78, 2.75, 1.75, 0.77}, {2.8, 2.0, 0.71, 1.8, 2.1, 1.0}},
+                    kCarry[2] = {{4.1, 4.4, 0.69, 0, 0.73, 0.92}, {2.8, 4.0, 0.72, 2.4, 0.9, 0.76}},
+                    kLarge[2] = {{3.0, 4.4, 2.27, 0, 0.8, 1.0}, {3.0, 4.4, 2.19, 0, 0.8, 1.1}};
+  const bool large = large_tiles(cus, M, N, carry);
+  const Cost &c = (M <= 32 ? k32 : large ? kLarge : carry ? kCarry : k64)[bt];
+  const int64_t mn = (int64_t)M * N;
+  const int64_t tiles = M <= 32 ? cdiv(M, 32) * cdiv(N, 128)
+                        : large ? cdiv(M, 128) * cdiv(N, 256) : cdiv(M, 64) * cdiv(N, 128);
+  const int steps = (int)cdiv(K, 32);
+  const int span = (int)cdiv(steps, pick_splits(tiles, steps, mn, cus)), s = (int)cdiv(steps, span);
+  const double us = c.fixed + 1e-6 * c.out * mn + (double)cdiv(tiles * s, cus) * (c.step * span + c.round) +
+                    (s > 1 ? c.split + 1e-6 * c.part * (s + 1) * mn : 0.) + 0.1 * std::min(K % 32, 8);
+  // rows of B_T that are whole 128 bytes apart meet in the same memory channels; a
+  // remainder of K is dearer yet to the fp32 MFMA kernels once they run many steps
+  return us * (K % 32 ? K < 256 && !bt ? 1.05 : 0.93 : bt ? 1.06 : 1.);
+}
 
 int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, int gs,
               const float *A, int64_t lda, float *C, int64_t ldc, int M, int K, float beta,
@@ -647,8 +678,7 @@ int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, 
   // waves, 22 on 32x64 of 4, 20 on 64x128)
   if (M <= 16) return X3_GO(1, 1, 4, 4);
   if (M <= 32) return X3_GO(2, 1, 8, 4);
-  // 128x256 tiles from two per CU on (4096^3: 686 us against 790 with 64x128)
-  if (carry && cdiv(M, 128) * cdiv(N, 256) >= 2 * num_cus()) return X3_GO(8, 2, 8, 2, true);
+  if (carry && large_tiles(num_cus(), M, N, carry)) return X3_GO(8, 2, 8, 2, true);
   if (carry) return X3_GO(4, 1, 8, 4, true);
   return X3_GO(4, 1, 8, 4);
 #undef X3_GO

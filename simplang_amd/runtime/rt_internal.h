@@ -238,6 +238,10 @@ int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, 
               const float *A, int64_t lda, float *C, int64_t ldc, int M, int K, float beta,
               bool must, bool carry, hipStream_t st);
 
+// Estimate in us of launch_x3's time for one fp32 product of more than 16 rows,
+// B[K,N] or B_T[N,K].
+double split_f32_us(int64_t cus, bool bt, int M, int N, int K, bool carry);
+
 // The tokens of a prompt, positions [p0, p0 + T), through all layers of the
 // decode engine at once (prefill.hip): fills the K/V cache rows of those
 // positions, as T steps would.

@@ -150,3 +150,30 @@ def test_w4_non_finite(dev):
     assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
     lim = _bound(K) * (np.abs(x[1]).astype(np.float64) @ np.abs(wd.T))
     assert (np.abs(got[1] - want[1]) <= lim).all()
+
+
+# aligned operands, where the dispatch chooses between the split products and the
+# fp32 MFMA kernels by their estimated times: sizes on both sides, 16, 30 and more
+# K parts, remainders of K, narrow C, one and several rounds of tiles
+CHOICE = [(17, 256, 8640), (33, 256, 4096), (64, 256, 8640), (64, 768, 768), (100, 1536, 900),
+          (128, 1024, 512), (200, 640, 2048), (256, 512, 132), (300, 3200, 260), (512, 4096, 48),
+          (1024, 128, 512), (1500, 1536, 1000), (2048, 32, 2048), (2048, 4096, 160)]
+
+
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("M,N,K", CHOICE)
+def test_f32_either_kernel(dev, M, N, K, nt):
+    import torch
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    a = torch.randn(M, K, device=dev, generator=g)
+    b = torch.randn(*((N, K) if nt else (K, N)), device=dev, generator=g)
+    c = torch.full((M + 1, N + 4), 7.0, device=dev)
+    (sa.tensor_matmul_nt_f32 if nt else sa.tensor_matmul_f32)(a, b, c[:M, :N])
+    bd = b.double().t().contiguous() if nt else b.double()
+    want = a.double() @ bd
+    # one rounding per product and sum at most (the fp32 MFMA kernels)
+    lim = (K + 40) * 2.0 ** -24 * (a.double().abs() @ bd.abs())
+    assert bool(((c[:M, :N] - want).abs() <= lim).all())
+    assert float((c[:M, :N] - want).norm() / want.norm()) <= 4 * 2.0 ** -24 * max(K, 16) ** 0.5
+    assert bool((c[M] == 7).all()) and bool((c[:, N:] == 7).all())
