@@ -693,7 +693,11 @@ int launch_gemm_t(const T *A, int64_t lda, int64_t sa, const T *B, int64_t ldb, 
     }
   }
   if constexpr (std::is_same<T, float>::value) {
-    if (batch == 1) {
+    // From four products a sum the split kernel is the closer one (1024x1024, K = 1,
+    // 2, 3, 4, 8, 32: 3.4e-8, 3.3e-8, 3.3e-8, 3.3e-8, 3.1e-8, 3.8e-8 off 64 bits in
+    // the 2-norm, gemm_t 2.5e-8, 3.1e-8, 3.6e-8, 4.0e-8, 5.4e-8, 1.0e-7; its largest
+    // error from four on too).
+    if (batch == 1 && K >= 4) {
       const X3Mat b{B, nullptr, N};
       const int rc = launch_x3(&b, 1, ldb, BT ? X3Fmt::kT : X3Fmt::kN, 0, 0, A, lda, C, ldc, M, K,
                                beta, true, true, st);

@@ -50,6 +50,25 @@ def test_f32_edges(dev, M, N, K, nt):
     assert (full[M] == 7).all() and (full[:, 0] == 7).all() and (full[:, N + 1:] == 7).all()
 
 
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("K", [1, 2, 3])
+def test_f32_shortest_sums(dev, K, nt):
+    """Sums of up to three products: one rounding each, by at most 2^-24 of what the
+    sum holds (K = 1: the rounded product)."""
+    import torch
+    g = torch.Generator(device=dev)
+    g.manual_seed(K)
+    a = torch.randn(1024, K + 1, device=dev, generator=g)[:, 1:]
+    b = torch.randn(*((1500, K) if nt else (K, 1500)), device=dev, generator=g)
+    c = torch.empty(1024, 1500, device=dev)
+    (sa.tensor_matmul_nt_f32 if nt else sa.tensor_matmul_f32)(a, b, c)
+    bd = b.double().t().contiguous() if nt else b.double()
+    lim = K * 2.0 ** -24 * (a.double().abs() @ bd.abs())
+    assert bool(((c - a.double() @ bd).abs() <= lim).all())
+    if K == 1:
+        assert torch.equal(c, a * (b.t() if nt else b))
+
+
 @pytest.mark.parametrize("M,N,K", [(40, 100, 70), (70, 130, 2050)])
 def test_f32_accumulates(dev, M, N, K):
     """``matmul`` adds to its output, with and without K splits."""
