@@ -1117,16 +1117,15 @@ __global__ void __launch_bounds__(256)
   C += blockIdx.z * sc;
   const int col = blockIdx.x * 64 + (threadIdx.x & 63);
   if (col >= N) return;
-  for (int row = blockIdx.y * 4 + (threadIdx.x >> 6); row < M; row += gridDim.y * 4) {
+  for (int64_t row = blockIdx.y * 4 + (threadIdx.x >> 6); row < M; row += gridDim.y * 4) {
     uint32_t s = 0;
     for (int k = 0; k < K; k++) {
-      const int32_t a = AU8 ? (int32_t)(uint8_t)A[(int64_t)row * lda + k]
-                            : (int32_t)A[(int64_t)row * lda + k];
+      const int32_t a = AU8 ? (int32_t)(uint8_t)A[row * lda + k] : (int32_t)A[row * lda + k];
       const int32_t b =
           BNK ? (int32_t)B[(int64_t)col * ldb + k] : (int32_t)B[(int64_t)k * ldb + col];
       s += (uint32_t)(a * b);
     }
-    C[(int64_t)row * ldc + col] = (int32_t)s;
+    C[row * ldc + col] = (int32_t)s;
   }
 }
 
@@ -1351,7 +1350,7 @@ int dispatch(const GemmArgs &g, hipStream_t st) {
     const int rc = dispatch_padded<BNK, AU8>(g, st);
     if (rc != 1) return rc;
   }
-  if ((!a_ok || !b_ok) && g.K >= 16 && (BNK || g.N >= 4))
+  if ((!a_ok || !b_ok) && g.K >= 16 && (BNK || g.N >= 4) && indexes_fit(g.M, g.N, g.K))
     return dispatch_tiles<BNK, AU8, true>(g, st);
   if (!a_ok || !b_ok) {
     dim3 grid((unsigned)cdiv(g.N, 64), (unsigned)std::min<int64_t>(cdiv(g.M, 4), 65535),

@@ -637,7 +637,7 @@ int launch_x3(const X3Mat *mats, int nmat, int64_t ldb, X3Fmt fmt, int64_t lds, 
               bool must, bool carry, hipStream_t st) {
   int64_t N = 0;
   for (int i = 0; i < nmat; i++) N += mats[i].n;
-  if (M <= 0 || N <= 0 || N > INT32_MAX || K <= 0 || nmat > 3) return 1;
+  if (M <= 0 || N <= 0 || K <= 0 || nmat > 3 || !indexes_fit(M, N, K)) return 1;
   // lane and row offsets of B[K,N] are 32-bit: 32 rows within 2 GiB
   if (fmt == X3Fmt::kN && ldb >= (int64_t(1) << 24)) return 1;
   X3Args a{};

@@ -132,6 +132,12 @@ int check_descn(const char *name, const void *aligned, int64_t off, int rank,
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Whether 32-bit row, column and K indices of a kernel that rounds sizes up to its
+// tiles and K spans (together less than 4096) stay below 2^31.
+constexpr bool indexes_fit(int64_t M, int64_t N, int64_t K) {
+  return M <= INT32_MAX - 4096 && N <= INT32_MAX - 4096 && K <= INT32_MAX - 4096;
+}
+
 // Number of CUs of the current device (cached per device).
 int num_cus();
 

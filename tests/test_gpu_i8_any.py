@@ -68,6 +68,25 @@ def test_padded_or_not(dev, M, N, K, nt):
     assert torch.equal(c, want.int())
 
 
+def test_rows_near_the_index_limit(dev):
+    """2^31 - 1 rows of 17 bytes: past what the tiled kernels index, on the generic
+    one, whose rows advance in steps of a grid."""
+    import torch
+    if torch.cuda.get_device_properties(dev).total_memory < 80 << 30:
+        pytest.skip("needs 45 GB")
+    M = 2 ** 31 - 1
+    a = torch.zeros((M, 17), dtype=torch.int8, device=dev)
+    rows = torch.tensor([0, 1, 262139, 2 ** 30, M - 262141, M - 2, M - 1], device=dev)
+    a[rows] = torch.arange(1, 8, dtype=torch.int8, device=dev)[:, None]
+    b = torch.full((1, 17), 3, dtype=torch.int8, device=dev)
+    c = torch.full((M, 1), 9, dtype=torch.int32, device=dev)
+    sa.tensor_matmul_nt_i8(a, b, c)
+    assert torch.equal(c[rows, 0], torch.arange(1, 8, dtype=torch.int32, device=dev) * 51)
+    assert int((c != 0).sum()) == 7
+    del a, c
+    torch.cuda.empty_cache()
+
+
 def test_any_batch(dev):
     import torch
     rng = np.random.default_rng(1)
