@@ -313,11 +313,12 @@ def f32_bench(dev, stream):
 
 
 def decode_bench(dev, stream, with_cpu=True):
-    """Greedy decode tok/s, BASELINE configs[3] (110M fp32) and configs[4]
-    (3B W4): random-init weights, random prompt of 32 tokens, then 256 / 128
-    greedy tokens, every step one replay of the captured step graph.  tok/s =
-    steps / wall time of the generation (one token per step, prompt steps
-    included, as bench_llama_quant.cpp:255-292 times every forward call)."""
+    """Greedy decode tok/s of the 110M fp32 and the 3B W4 model: random-init
+    weights, random prompt of 32 tokens, then 256 / 128 greedy tokens, every one
+    of them one replay of the captured step graph.  tok/s = generated tokens over
+    the wall time of their steps (as bench_llama_quant.cpp:255-292 times every
+    forward call); the prompt before its last token, which the engine takes
+    through the layers in one pass, is timed on its own and counts in neither."""
     import numpy as np
     import torch
     import simplang_amd as sa
@@ -330,20 +331,26 @@ def decode_bench(dev, stream, with_cpu=True):
         # capture + warm: the same positions as the timed run, so every step
         # graph (one per attention form and chunk count) exists before timing
         m.generate(prompt, n_new, use_graph=True)
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        toks = m.generate(prompt, n_new, use_graph=True)
-        el = time.perf_counter() - t0
-        steps = len(prompt) + n_new - 1
+
+        def timed(n):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            toks = m.generate(prompt, n, use_graph=True)
+            return time.perf_counter() - t0, toks
+
+        pre = min(timed(0)[0] for _ in range(3))  # all of the prompt but its last token
+        el, toks = timed(n_new)
+        el -= pre
+        first = len(prompt) - 1   # position of the first step: the last prompt token
         m.close()
-        byts = np.mean([weight_bytes(cfg) + kv_bytes(cfg, p) for p in range(steps)])
-        rec = {"model": name, "prompt": 32, "generated": n_new, "tok_s": round(steps / el, 1),
-               "ms_per_token": round(el / steps * 1e3, 3),
-               "GBs": round(byts * steps / el / 1e9, 1),
-               "frac_hbm": round(byts * steps / el / 1e9 / HBM_PEAK_GBS, 3),
+        byts = np.mean([weight_bytes(cfg) + kv_bytes(cfg, first + i) for i in range(n_new)])
+        rec = {"model": name, "prompt": 32, "prompt_ms": round(pre * 1e3, 3), "generated": n_new,
+               "tok_s": round(n_new / el, 1), "ms_per_token": round(el / n_new * 1e3, 3),
+               "GBs": round(byts * n_new / el / 1e9, 1),
+               "frac_hbm": round(byts * n_new / el / 1e9 / HBM_PEAK_GBS, 3),
                "tokens_head": [int(t) for t in toks[32:40]]}
         if with_cpu:
-            rec["cpu_baseline"] = decode_cpu(cfg, w, prompt, steps)
+            rec["cpu_baseline"] = decode_cpu(cfg, w, prompt, first, n_new)
         out.append(rec)
         del w
         torch.cuda.empty_cache()
@@ -517,20 +524,20 @@ def llama2_quant_bench(dev, with_cpu=True):
     return out
 
 
-def decode_cpu(cfg, w, prompt, n_steps, sample_steps=20):
+def decode_cpu(cfg, w, prompt, first, n_steps, sample_steps=20):
     """The decode CPU baseline (oracle/cpu_decode.c: the step restated in fp32,
     OpenMP GEMVs over output rows in 16 fp32 lanes, the host cores one GPU gets)
     on a bounded sample of the same generation: `sample_steps` consecutive
-    steps centred on the mean position of the GPU run's `n_steps`, the cache
-    rows below the first one filled with random values (the work of a step does
-    not depend on what the rows hold).  tok/s = steps / wall time of that loop
-    (bench_llama_quant.cpp:255-292)."""
+    steps centred on the mean position of the GPU run's `n_steps` from position
+    `first` on, the cache rows below the first one filled with random values
+    (the work of a step does not depend on what the rows hold).  tok/s = steps /
+    wall time of that loop (bench_llama_quant.cpp:255-292)."""
     import numpy as np
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
     import oracle
     wn = {k: v.detach().cpu().numpy() for k, v in w.items()}
     o = oracle.CpuLlama(cfg, wn)
-    p0 = max(0, (n_steps - 1) // 2 - sample_steps // 2)
+    p0 = max(0, first + (n_steps - 1) // 2 - sample_steps // 2)
     kv = cfg["dim"] * cfg["n_kv_heads"] // cfg["n_heads"]
     rng = np.random.default_rng(5)
     for c in (o.kc, o.vc):
