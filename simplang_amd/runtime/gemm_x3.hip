@@ -141,8 +141,14 @@ struct X3Args {
 //     the nibble conversion and the scaling (200x3200x8640: 58 us; one thread
 //     per output took 131 ms).
 //   * A part that overflows or an infinite or NaN operand makes its products
-//     NaN where fp32 arithmetic may give an infinity: tiles with a non-finite
-//     sum are formed again with v_mfma_f32_16x16x4_f32 from the fp32 operands.
+//     NaN where fp32 arithmetic may give an infinity: 16x16 tiles with a
+//     non-finite sum are formed again with v_mfma_f32_16x16x4_f32 from the fp32
+//     operands, without LDS.  Both operands are scaled by 2^24, so that happens to
+//     finite products too, where a sum on its way reaches 2^80 (W4: 2^104 before
+//     its scale) or an operand 2^104.  It costs: 4096^3 0.58 ms, with one infinity
+//     in A 1.46 and in B 0.81 (6.0 and 4.9 when whole tiles of a wave were formed
+//     again), with all sums beyond 8.0, where the fp32 MFMA kernel takes 1.02
+//     whatever the values.
 template <int MT, int NT, int NW, int KIND, int PD, bool CARRY = false, int PA = 2>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
     gemm_x3(const X3Args a) {
@@ -447,27 +453,47 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
       for (int e = 0; e < 4; e++) bad |= !(fabsf(acc[i][j][e]) <= 3.4028235e38f);
   if (__builtin_expect(__any(bad), 0)) {
+    uint32_t which = 0;  // 16x16 tiles of this wave
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        bool b16 = false;
+#pragma unroll
+        for (int e = 0; e < 4; e++) b16 |= !(fabsf(acc[i][j][e]) <= 3.4028235e38f);
+        if (__any(b16)) which |= 1u << (i * NT + j);
+      }
 #pragma unroll 1
     for (int t = 0; t < MT * NT; t++) {
+      if (!(which >> t & 1)) continue;
       const int ti = t / NT, tj = t - ti * NT;
       const float *ap = a.A + (int64_t)min(m0 + 16 * ti + r16, a.M - 1) * a.lda;
       const int n = min(n0 + 16 * tj + r16, b.n - 1);
-      v4f c = {0.f, 0.f, 0.f, 0.f};
-      for (int k = 32 * s0; k < kend; k += 4) {
-        const int kk = k + g;
-        float av = 0.f, bv = 0.f;
-        if (kk < kend) {
-          av = ap[kk];
-          if constexpr (KIND == kBKN) bv = ((const float *)b.B)[(int64_t)kk * a.ldb + n];
-          if constexpr (KIND == kBNK) bv = ((const float *)b.B)[(int64_t)n * a.ldb + kk];
-          if constexpr (W4) {
-            const uint8_t w = ((const uint8_t *)b.B)[(int64_t)n * a.ldb + (kk >> 1)];
-            const int q = (int)((uint32_t)w << (kk & 1 ? 24 : 28)) >> 28;
-            bv = (float)q * b.S[(int64_t)n * a.lds + chunk_group(kk >> 5, a.cpg, a.cpg_shift)];
-          }
+      auto bat = [&](int kk) {
+        if constexpr (KIND == kBKN) return ((const float *)b.B)[(int64_t)kk * a.ldb + n];
+        if constexpr (KIND == kBNK) return ((const float *)b.B)[(int64_t)n * a.ldb + kk];
+        if constexpr (W4) {
+          const uint8_t w = ((const uint8_t *)b.B)[(int64_t)n * a.ldb + (kk >> 1)];
+          const int q = (int)((uint32_t)w << (kk & 1 ? 24 : 28)) >> 28;
+          return (float)q * b.S[(int64_t)n * a.lds + chunk_group(kk >> 5, a.cpg, a.cpg_shift)];
         }
+      };
+      v4f c = {0.f, 0.f, 0.f, 0.f};
+      auto mul = [&](float av, float bv) {
         c = W4 ? __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, c, 0, 0, 0)
                : __builtin_amdgcn_mfma_f32_16x16x4f32(bv, av, c, 0, 0, 0);
+      };
+      int k = 32 * s0;
+      for (; k + 32 <= kend; k += 32) {  // eight loads of each operand in flight
+        float av[8], bv[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) av[u] = ap[k + 4 * u + g], bv[u] = bat(k + 4 * u + g);
+#pragma unroll
+        for (int u = 0; u < 8; u++) mul(av[u], bv[u]);
+      }
+      for (; k < kend; k += 4) {
+        const bool in = k + g < kend;
+        mul(in ? ap[k + g] : 0.f, in ? bat(k + g) : 0.f);
       }
 #pragma unroll
       for (int i = 0; i < MT; i++)
