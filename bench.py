@@ -2,7 +2,7 @@
 """Benchmark of libsimp_hip.so on one MI355X.
 
 Headline (the JSON line's ``value``): exact int8 GEMM throughput, u8 x s8 -> i32
-(vpdpbusd semantics), at the largest square shape of BASELINE configs[1]
+(vpdpbusd semantics), at the largest square shape of the int8 sweep
 (8192^3), inputs resident in HBM.  One step = one C = A x B over the
 synthetic batch (A u8 uniform [0,255], B s8 uniform [-128,127], seed 42).
 
@@ -18,7 +18,7 @@ recover over its first ~60 calls (per-call times on one box: 546, 601, 652,
 the K timed ones; the line reports the count as ``settle_calls``.  Without
 them, 5 warmup + 20 timed calls average 613 us on the same box.
 
-Also reported on the same line: the configs[1] sweep (TOPS per shape), the W4
+Also reported on the same line: the int8 sweep (TOPS per shape), the W4
 GEMV (with its CPU baseline per shape), rmsnorm / softmax / silu, fp32 GEMM and
 decode sections, and the CPU baseline -- the oracle's restatement of the
 reference's VNNI kernel timed on the host cores one GPU gets (and on one core)
@@ -73,7 +73,7 @@ def make_inputs(M, N, K, dev, seed=42):
     return a, b, c
 
 
-# One MI355X's share of its box's host CPUs: the GPU boxes give each GPU 16
+# One MI355X's share of its host's CPUs: each GPU is given 16
 # cores whatever nproc reports, so "all cores" means at most 16 there.
 CPU_SHARE = 16
 
@@ -191,7 +191,7 @@ def w4_cpu_us(w, s, x, threads, budget_s=0.4):
 
 
 def w4_bench(dev, stream, with_cpu=True):
-    """W4 GEMV/skinny GEMM, BASELINE configs[2].  Weight copies are rotated so
+    """W4 GEMV/skinny GEMM at the 3B model's shapes.  Weight copies are rotated so
     that more than 512 MB is touched per pass: every launch streams its weights
     from HBM (the 256 MB Infinity Cache cannot hold them), as in a decode step.
     Timed by HIP-graph replay of one launch per copy.  Each row also carries the
@@ -682,7 +682,7 @@ def main():
         "vs_baseline": None,
         "dtype": "int8 (u8 x s8 -> i32)",
         "data": "synthetic: A u8 uniform [0,255], B s8 uniform [-128,127], seed 42",
-        "config": {"workload": f"int8 GEMM u8xs8->i32 {n}^3 (BASELINE configs[1], largest square)",
+        "config": {"workload": f"int8 GEMM u8xs8->i32 {n}^3 (largest square of the sweep)",
                    "M": n, "N": n, "K": n, "layout": "A[M,K], B[K,N] row-major, C[M,N] i32"},
         "roofline": {"bound": "mfma", "achieved": round(ktops, 2), "peak": INT8_PEAK_TOPS,
                      "unit": "TFLOP/s", "frac": round(ktops / INT8_PEAK_TOPS, 4),

@@ -58,7 +58,12 @@ const char *simp_rt_last_error(void);
 int64_t simp_rt_error_count(void);
 int32_t simp_rt_version(void);
 int32_t simp_rt_init(void);
-int32_t simp_rt_set_stream(void *hip_stream); /* per calling thread; NULL = null stream */
+/* Per calling thread; NULL = null stream.  Several threads may use one stream.  A
+ * call that needs device scratch under stream capture uses what an uncaptured call
+ * of the same size on that stream has left; graphs recorded on one stream share
+ * it, so their replays must not overlap each other (they may overlap anything
+ * else). */
+int32_t simp_rt_set_stream(void *hip_stream);
 void *simp_rt_get_stream(void);
 int32_t simp_rt_sync(void);
 int32_t simp_rt_register(const void *host_ptr, int64_t bytes, int32_t flags);

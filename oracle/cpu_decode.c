@@ -3,7 +3,7 @@
  * cpu_baseline leg only (TEST INFRASTRUCTURE: never on the product path;
  * tests/test_oracle_decode.py checks it against orc_llama_forward).
  *
- * One token of stories110M.sl:44-247 (fp32 weights) or of the BASELINE W4
+ * One token of stories110M.sl:44-247 (fp32 weights) or of the symmetric W4
  * model (every linear weight signed nibbles in [-8,7], one fp32 scale per group
  * of gs along K, the matmul_quant loop of ConvertSimpToMemRef.cpp:3906-4005 with
  * the signed nibbles of :3016-3037), in fp32 throughout as the compiled program

@@ -1,12 +1,11 @@
 """ctypes wrapper of the CPU oracle (oracle/_build/liboracle.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and
-bench.py's cpu_baseline leg, as the checker.  Nothing on the product path
+bench.py's cpu_baseline leg, as the oracle.  Nothing on the product path
 imports it.  The optional in-place reference build (oracle/_ref/libsimpref.so,
-only where the SimpLang sources are mounted in this container) is loaded only on
-request, by ``load_ref()`` (None when it is not built).  It is listed in
-.gpurunignore: it never travels to the GPU box, and no GPU test, smoke() or
-bench.py loads it.
+only where the SimpLang sources are mounted) is loaded only on request, by
+``load_ref()`` (None when it is not built); no GPU test, smoke() or bench.py loads
+it.
 """
 from __future__ import annotations
 

@@ -1211,8 +1211,10 @@ int capture_step(LlamaModel &m, int mode) {
 // Runs the first n tokens of the prompt (already on the device) as rows of
 // matrices; *done receives how many of them it took, n or 0 (shapes or weights
 // that the row kernels do not take, no memory for the activations, or too few
-// tokens: the steps then take the prompt, writing every cache row again; a pass costs about as much as five steps: 110M 1.4 ms for 199 tokens, 3B W4
-// 4.4 ms for 31, against 0.31 and 0.88 ms a step).
+// tokens: the steps then take the prompt, writing every cache row again).  A pass
+// costs about as much as three to five steps (110M 0.8 ms for 31 tokens, 1.4 for
+// 199; 3B W4 3.7 ms for 31; 0.31 and 0.88 ms a step): with nine prompt tokens, a pass
+// and a step against nine steps, 0.91 against 2.57 ms and 4.2 against 7.8.
 constexpr int64_t kPrefillMin = 8, kPrefillRows = 512;
 int prefill_prompt(LlamaModel &m, int64_t n, int64_t *done) {
   *done = 0;

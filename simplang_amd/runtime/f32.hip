@@ -9,9 +9,10 @@
 // n == 1 (every LLaMA decode projection, stories110M.sl:77-83) is an HBM-bound
 // GEMV: one wave per output row at a time, lanes along K with 16-byte loads, x
 // held in registers for the whole kernel, the next row's loads in flight while
-// the current row is reduced.  Single products of more than 16 rows, or with
-// operands that 16-byte loads cannot read, run on the split-bf16 kernel
-// (gemm_x3.hip); batches and few rows on the fp32 MFMA kernels here.
+// the current row is reduced.  Single products with
+// operands that 16-byte loads cannot read run on the split-bf16 kernel
+// (gemm_x3.hip), and aligned ones of more than 16 rows where it is the faster one;
+// the others, batches and few rows on the fp32 MFMA kernels here.
 #include <algorithm>
 #include <type_traits>
 

@@ -30,9 +30,12 @@
 //     the u8 column sums come from the B fragments in registers (v_dot4
 //     against 0x01010101).  Skinny problems split K over grid y and combine
 //     partial tiles with integer atomics into a zero-filled C (exact).
-//   * gemm_i8_generic -- operands the MFMA kernels cannot load with aligned
-//     vector loads (K % 16 != 0, N % 4 != 0 for B[K,N], misaligned bases): one
-//     output element per thread.
+//   * gemm_i8_mfma with ANY -- operands that aligned vector loads cannot read (K %
+//     16 != 0, N % 4 != 0 for B[K,N], misaligned rows): the same tiles on
+//     byte-aligned loads, from K = 16 (N = 4 for B[K,N]) on.  Large products of such
+//     operands go through padded copies to the kernels for B_T (dispatch_padded).
+//   * gemm_i8_generic -- what is left: fewer k-rows or columns than one load, and
+//     sizes within a few thousand of 2^31; one output element per thread.
 // Workgroup ids are remapped so that each of the 8 XCDs owns a contiguous range
 // of tiles (blocks are dispatched round-robin over XCDs), and tiles are ordered
 // in groups of 8 tile-rows so co-resident tiles share A and B in L2.
@@ -660,8 +663,8 @@ __global__ void __launch_bounds__(512)
 #pragma unroll
     for (int j = 0; j < FN; j++) {
       const int col = n0 + wn0 + 16 * (j ^ jx) + 4 * lkc;
-      // u8 x s8: C = (A^0x80) B + 128 colsum(B)
-      // (N % 16 == 0 and col % 4 == 0, so col < N covers col..col+3)
+      // u8 x s8: C = (A^0x80) B + 128 colsum(B).  (colsum[] comes from a pass over B
+      // that is only dispatched with N % 16 == 0, where col < N covers col..col+3)
       v4i bias = v4i{0, 0, 0, 0};
       if constexpr (CS) {
         bias = cs_lds[(wn0 + 16 * (j ^ jx)) / 4 + lkc] * 128;
@@ -1104,9 +1107,9 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Correctness fallback for shapes the MFMA path cannot load with aligned
-// vector loads (K % 16 != 0, N % 4 != 0 for B[K,N], misaligned bases).  Rows
-// stride over grid y; z is the batch.
+// One output element per thread, for what the MFMA tiles do not take: unaligned
+// operands with K < 16 (or N < 4 for B[K,N]), sizes next to 2^31.  Rows stride over
+// grid y; z is the batch.
 template <bool BNK, bool AU8>
 __global__ void __launch_bounds__(256)
     gemm_i8_generic(const int8_t *__restrict__ A, int64_t lda, const int8_t *__restrict__ B,

@@ -2,13 +2,20 @@
 //
 // Every fp32 operand is split into three bf16 parts, x = h + m + l exactly (8 +
 // 8 + 8 significant bits: h = bf16(x), m = bf16(x - h), l = x - h - m), whose
-// products are exact in fp32.  A product of two fp32 values keeps the six parts
-// hh, hm, mh, hl, lh and mm; the three dropped ones are below 2^-25 of it, less
-// than one fp32 rounding.  A W4 weight is one exact bf16, so there the three
-// products are all of them.  v_mfma_f32_16x16x32_bf16 runs at 16 times the rate
-// of v_mfma_f32_16x16x4_f32 and rounds its accumulator once per 32 products
-// instead of once per 4, so six of them are faster than the fp32 MFMA and no
-// less exact.
+// products are exact in fp32 (the splitting of G. Henry, P. Tang and A. Heinecke,
+// "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019).  A product of two fp32 values keeps the six parts
+// hh, hm, mh, hl, lh and mm; each of the three dropped ones is below 2^-25 of it,
+// together they reach 2^-24, half a unit of fp32, at most.  A W4 weight is one
+// exact bf16, so there the three products are all of them.
+// v_mfma_f32_16x16x32_bf16 runs at 16 times the rate of v_mfma_f32_16x16x4_f32 and
+// rounds its accumulator once per 32 products instead of once per 4: six of them
+// take less time than the fp32 MFMA, and from four products a sum on come closer to
+// 64 bits than the fp32 kernels (K = 4 / 32 / 128 / 512, closed every step 3.3e-8 /
+// 3.7e-8 / 5.5e-8 / 7.0e-8 off in the 2-norm, carried 3.2e-8 / 3.8e-8 / 1.5e-7 /
+// 3.4e-7, fp32 MFMA or FMA 4.0e-8 / 1.0e-7 / 2.0e-7 / 4.1e-7).  What they do
+// not have is a mean error of zero: up to one step, where no sign has turned
+// yet, it is 0.16 to 0.35 of the root mean square one, towards smaller values.
 #include <algorithm>
 #include <type_traits>
 
@@ -132,12 +139,13 @@ struct X3Args {
 //   * Nothing depends on the alignment of any operand beyond its type's
 //     (W4: rows of 4-byte aligned bytes).  Rows past M and columns past N read
 //     the last one and are not stored; only the last step reads under a mask.
-//   * What bounds it: large products the MFMA rate the chip sustains (4096^3: 686
-//     us against 1020 for the fp32 MFMA kernel; the MFMA pipe is busy 65% of the
-//     cycles at 1.75 GHz, 1.2 PFLOP/s of bf16, where a bf16 library GEMM reaches
-//     1.1 to 1.4); mid sizes the splitting next to it (128x2048x8192 32.8 us
-//     against 43.0, 301x1537x2003 with B_T 23.4 against 314 for the SIMT kernel
-//     that odd sizes took; a copy without the operand loads runs as long).  W4:
+//   * What bounds it: large products the MFMA rate the chip sustains (4096^3: 580
+//     to 690 us from card to card against 1020 for the fp32 MFMA kernel; the MFMA pipe
+//     is busy 65% of the cycles at 1.75 GHz, 1.2 PFLOP/s of bf16, where a bf16
+//     library GEMM reaches 1.1 to 1.4); mid sizes the splitting next to it
+//     (128x2048x8192 32.8 us against 43.0, 301x1537x2003 with B_T 23.1 against 227
+//     for the SIMT kernel that odd sizes took; a copy without the operand loads
+//     runs as long).  W4:
 //     the nibble conversion and the scaling (200x3200x8640: 58 us; one thread
 //     per output took 131 ms).
 //   * A part that overflows or an infinite or NaN operand makes its products
@@ -567,8 +575,7 @@ __global__ void __launch_bounds__(256)
 // CUs costs its steps and about four more to fill and drain its pipeline; the
 // partial sums cost a launch (about three steps' time) and their traffic (a
 // step is about 1 us, in which 4 MB go by).  Measured (W4, 200 x 3200 -> 8640,
-// 68 tiles: 3 / 6 / 7 splits 61 / 72 / 71 us; fp32 128 x 2048 x 8192,
-// 128 tiles: 1 / 2 / 4 splits 70 / 39 / 39 us).  More than 16 splits only within
+// 68 tiles: 3 / 6 / 7 splits 61 / 72 / 71 us).  More than 16 splits only within
 // one round (64x256x8640, 2 tiles: 16 / 30 splits 19.7 / 14.8 us).
 int pick_splits(int64_t tiles, int steps, int64_t mn, int64_t cus) {
   int best = 1;

@@ -116,7 +116,7 @@ def test_one_block_attention_head_size_over_128(dev, orc):
 
 
 def test_110m_f32_greedy_256(dev, orc):
-    """32-token random prompt, 256 greedy tokens."""
+    """110M fp32: 32-token random prompt, 256 greedy tokens."""
     cfg = CFG_110M
     w = make_model(cfg, dev, seed=42)
     prompt = np.random.default_rng(42).integers(0, cfg["vocab_size"], 32).astype(np.int32)
@@ -134,7 +134,7 @@ def test_110m_f32_greedy_256(dev, orc):
 
 
 def test_3b_w4_logits_and_greedy(dev, orc):
-    """BASELINE configs[4] at full size: logits at 3 positions and 16 greedy
+    """3B W4 at full size: logits at 3 positions and 16 greedy
     steps through the captured step graphs (the oracle needs ~1 s per 3B step
     on the host)."""
     import torch
@@ -154,7 +154,7 @@ def test_3b_w4_logits_and_greedy(dev, orc):
 
 
 def test_3b_dims_two_layers_every_chunk_count(dev, orc):
-    """The kernels the configs[4] bench times, at its dims (dim 3200, 32 heads
+    """The kernels the 3B W4 bench times, at its dims (dim 3200, 32 heads
     of 100, hidden 8640, W4 g32) with 2 layers and a smaller vocabulary: logits
     at every position 0..319 (attention over 1, 2, 3, 4 chunks of 64 with the
     combine folded into the Wo GEMV, then 5 chunks with the separate combine),

@@ -1,6 +1,6 @@
 """GPU parity of the int8 GEMM entry points against the pinned oracle.
 
-Bit-exact for every shape (integer arithmetic).  Full BASELINE sizes that the
+Bit-exact for every shape (integer arithmetic).  Full benchmark sizes that the
 CPU oracle cannot finish in seconds (4096^3, 8192^3) are checked through
 size-independent identities: row sums C*1 = A*(B*1), column sums 1^T*C =
 (1^T*A)*B (exact in int64), a sample of full rows recomputed exactly, and the

@@ -1,7 +1,7 @@
 """GPU side of the model files: the llama2.c checkpoint loaded into device
 memory (generate_stories110M.cpp:150-191), the W4 quantizers against the
 oracle's restatements bit for bit (reference quantize_w4,
-bench_llama_quant.cpp:51-93, and the symmetric BASELINE format), and the packed
+bench_llama_quant.cpp:51-93, and the symmetric format), and the packed
 W4 files written from a checkpoint and read back, driven through the decode
 engine and llama2_quant_forward against the oracle's forward passes."""
 import numpy as np

@@ -1,7 +1,7 @@
 """GPU parity of the fp32 ops (matmul, tensor_matmul f32, rmsnorm, softmax,
 silu, swiglu, rope) against the pinned oracle and the reference's KATs.
 
-Tolerance (BASELINE: fp32 within 1e-4 relative): max|gpu - ref| <= 1e-4 *
+Tolerance (fp32 within 1e-4 relative): max|gpu - ref| <= 1e-4 *
 max|ref| per output vector, ref being the oracle (matmuls: float64).
 """
 import numpy as np
@@ -201,7 +201,7 @@ def test_rope_vs_oracle(dev, orc, dim, kv_dim, hs, pos):
     orc.rope(qo, ko, dim, kv_dim, hs, pos)
     # fp32 angles as in the reference (float literals are f32, mlir_codegen.cpp:608-626):
     # a 1-ulp powf difference between device and host libm grows with pos (~500 rad),
-    # so RoPE is held to the BASELINE tolerance, 1e-4.
+    # so RoPE is held to the path's tolerance, 1e-4.
     _close(tq.cpu().numpy(), qo)
     _close(tk.cpu().numpy(), ko[:kv_dim])
 

@@ -1,7 +1,7 @@
 """GPU parity of the W4 GEMV / skinny GEMM entry points against the oracle.
 
 fp32 results are compared with the oracle's double-precision value of the same
-dequantised product.  Tolerance (written here, from BASELINE's 1e-4 relative):
+dequantised product.  Tolerance (written here, from the path's 1e-4 relative):
 normwise  max|gpu - ref| <= 1e-4 * max|ref|  for every output row of x.
 """
 import numpy as np
@@ -15,7 +15,7 @@ TOL = 1e-4
 
 
 def _w4s_inputs(M, N, K, gs, seed):
-    """q uniform in [-8,7], scale |N(0,0.02)|/7 per group, x ~ N(0,1)."""
+    """The W4 benchmark's inputs: q uniform in [-8,7], scale |N(0,0.02)|/7 per group, x ~ N(0,1)."""
     rng = np.random.default_rng(seed)
     q = rng.integers(-8, 8, (N, K))
     nib = (q & 15).astype(np.uint8)
