@@ -61,8 +61,8 @@ int32_t simp_rt_init(void);
 /* Per calling thread; NULL = null stream.  Several threads may use one stream.  A
  * call that needs device scratch under stream capture uses what an uncaptured call
  * of the same size on that stream has left; graphs recorded on one stream share
- * it, so their replays must not overlap each other (they may overlap anything
- * else). */
+ * it, so their replays must not overlap each other, nor what was launched on that
+ * stream before the capture (they may overlap anything else). */
 int32_t simp_rt_set_stream(void *hip_stream);
 void *simp_rt_get_stream(void);
 int32_t simp_rt_sync(void);
